@@ -2,7 +2,7 @@
 //
 // One wavefront (64 lanes) owns S complex sequences of length N held in its
 // own slice of LDS; stages exchange data through that slice with wavefront
-// ordering only (no workgroup barrier).  A group of LN = 128, 192, ... lanes
+// ordering only (no workgroup barrier).  A group of LN = 128, ... lanes
 // (consecutive wavefronts of a workgroup) can share the sequences instead:
 // its stages are ordered by the workgroup barrier, so every wavefront of the
 // workgroup runs the same stages.  Lengths, radices and stage strides
@@ -94,24 +94,22 @@ struct Dft<4, SIGN> {
     }
 };
 
-// 6 = 2 x 3: X[k] = E[k%3] + w^k O[k%3], X[k+3] = E[k] - w^k O[k], w = exp(SIGN pi i / 3)
+// 6 = 2 x 3 by the prime-factor map (n = 3 n1 + 2 n2, k = 3 k1 + 4 k2 mod 6:
+// n k = 3 n1 k1 + 2 n2 k2 mod 6), so no factor stands between the 3-point and
+// the 2-point transforms
 template <int SIGN>
 struct Dft<6, SIGN> {
     template <class C>
     __device__ static inline void run(C *v) {
-        using T = typename CxT<C>::R;
-        C e[3] = {v[0], v[2], v[4]}, o[3] = {v[1], v[3], v[5]};
+        C e[3] = {v[0], v[2], v[4]}, o[3] = {v[3], v[5], v[1]};
         Dft<3, SIGN>::run(e);
         Dft<3, SIGN>::run(o);
-        const T s = T(SIGN * 0.86602540378443864676), h = T(0.5);
-        const C o1 = mkc<C>(h * o[1].x - s * o[1].y, h * o[1].y + s * o[1].x);
-        const C o2 = mkc<C>(-h * o[2].x - s * o[2].y, -h * o[2].y + s * o[2].x);
         v[0] = cadd(e[0], o[0]);
         v[3] = csub(e[0], o[0]);
-        v[1] = cadd(e[1], o1);
-        v[4] = csub(e[1], o1);
-        v[2] = cadd(e[2], o2);
-        v[5] = csub(e[2], o2);
+        v[4] = cadd(e[1], o[1]);
+        v[1] = csub(e[1], o[1]);
+        v[2] = cadd(e[2], o[2]);
+        v[5] = csub(e[2], o[2]);
     }
 };
 
@@ -139,6 +137,93 @@ struct Dft<8, SIGN> {
     }
 };
 
+// z * exp(SIGN 2 pi i m / n) for a literal cosine and sine of 2 pi m / n
+template <int SIGN, class C>
+__device__ inline C rot(C z, typename CxT<C>::R c, typename CxT<C>::R s) {
+    using T = typename CxT<C>::R;
+    const T t = T(SIGN) * s;
+    return mkc<C>(z.x * c - z.y * t, z.x * t + z.y * c);
+}
+
+// 9 = 3 x 3: n = 3 n1 + n2, k = k1 + 3 k2, w = exp(SIGN 2 pi i / 9) on n2 k1
+template <int SIGN>
+struct Dft<9, SIGN> {
+    template <class C>
+    __device__ static inline void run(C *v) {
+        C a[3] = {v[0], v[3], v[6]}, b[3] = {v[1], v[4], v[7]}, c[3] = {v[2], v[5], v[8]};
+        Dft<3, SIGN>::run(a);
+        Dft<3, SIGN>::run(b);
+        Dft<3, SIGN>::run(c);
+        b[1] = rot<SIGN>(b[1], 0.76604444311897803520, 0.64278760968653932632);    // 1/9 turn
+        b[2] = rot<SIGN>(b[2], 0.17364817766693034885, 0.98480775301220805937);    // 2/9
+        c[1] = rot<SIGN>(c[1], 0.17364817766693034885, 0.98480775301220805937);    // 2/9
+        c[2] = rot<SIGN>(c[2], -0.93969262078590838405, 0.34202014332566873304);   // 4/9
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            C t[3] = {a[k], b[k], c[k]};
+            Dft<3, SIGN>::run(t);
+            v[k] = t[0];
+            v[k + 3] = t[1];
+            v[k + 6] = t[2];
+        }
+    }
+};
+
+// 12 = 3 x 4 by the prime-factor map: n = 4 n1 + 3 n2, k = 4 k1 + 9 k2 mod 12
+template <int SIGN>
+struct Dft<12, SIGN> {
+    template <class C>
+    __device__ static inline void run(C *v) {
+        C y[4][3];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < 3; ++n1) y[n2][n1] = v[(4 * n1 + 3 * n2) % 12];
+            Dft<3, SIGN>::run(y[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < 3; ++k1) {
+            C t[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
+            Dft<4, SIGN>::run(t);
+#pragma unroll
+            for (int k2 = 0; k2 < 4; ++k2) v[(4 * k1 + 9 * k2) % 12] = t[k2];
+        }
+    }
+};
+
+// 16 = 4 x 4: n = 4 n1 + n2, k = k1 + 4 k2, w = exp(SIGN 2 pi i / 16) on n2 k1
+template <int SIGN>
+struct Dft<16, SIGN> {
+    template <class C>
+    __device__ static inline void run(C *v) {
+        using T = typename CxT<C>::R;
+        const T h = T(0.70710678118654752440), c1 = T(0.92387953251128675613), s1 = T(0.38268343236508977173);
+        C y[4][4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < 4; ++n1) y[n2][n1] = v[4 * n1 + n2];
+            Dft<4, SIGN>::run(y[n2]);
+        }
+        y[1][1] = rot<SIGN>(y[1][1], c1, s1);      // 1/16 turn
+        y[1][2] = rot<SIGN>(y[1][2], h, h);        // 2/16
+        y[1][3] = rot<SIGN>(y[1][3], s1, c1);      // 3/16
+        y[2][1] = rot<SIGN>(y[2][1], h, h);        // 2/16
+        y[2][2] = mul_si<SIGN>(y[2][2]);           // 4/16
+        y[2][3] = rot<SIGN>(y[2][3], -h, h);       // 6/16
+        y[3][1] = rot<SIGN>(y[3][1], s1, c1);      // 3/16
+        y[3][2] = rot<SIGN>(y[3][2], -h, h);       // 6/16
+        y[3][3] = rot<SIGN>(y[3][3], -c1, -s1);    // 9/16
+#pragma unroll
+        for (int k1 = 0; k1 < 4; ++k1) {
+            C t[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
+            Dft<4, SIGN>::run(t);
+#pragma unroll
+            for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = t[k2];
+        }
+    }
+};
+
 // exp(SIGN 2 pi i m / N) from the table tw[k] = exp(-2 pi i k / N)
 template <int SIGN, class C>
 __device__ inline C twiddle(const C *__restrict__ tw, int m) {
@@ -157,10 +242,15 @@ __device__ inline void twiddle_powers(const C *__restrict__ tw, int m, C (&p)[R]
     if constexpr (std::is_same<C, float2>::value) {
 #pragma unroll
         for (int r = 1; r < R; ++r) p[r] = twiddle<SIGN>(tw, r * m);
-    } else {
+    } else if constexpr (R <= 8) {
         p[1] = twiddle<SIGN>(tw, m);
 #pragma unroll
         for (int r = 2; r < R; ++r) p[r] = cmul(p[r - 1], p[1]);
+    } else {
+        p[1] = twiddle<SIGN>(tw, m);
+#pragma unroll
+        for (int r = 2; r < R; ++r)
+            p[r] = r % 4 == 0 ? twiddle<SIGN>(tw, r * m) : cmul(p[r - 1], p[1]);
     }
 }
 
@@ -262,18 +352,6 @@ struct GStagesLSW<LN, N, SIGN, S, LS, WI, SW, NS, R, Rs...> {
 // one wavefront per group of sequences
 template <int N, int SIGN, int S, int LS, int WI, bool SW, int NS, int... Rs>
 using StagesLSW = GStagesLSW<64, N, SIGN, S, LS, WI, SW, NS, Rs...>;
-// contiguous sequences shared by LN lanes, unswizzled
-template <int LN, int N, int SIGN, int S, int NS, int... Rs>
-using GStages = GStagesLSW<LN, N, SIGN, S, N, 0, false, NS, Rs...>;
-
-// runs on unswizzled input, without (StagesLS) or with (StagesLSZ) swizzled writes
-template <int N, int SIGN, int S, int LS, int NS, int... Rs>
-using StagesLS = StagesLSW<N, SIGN, S, LS, 0, false, NS, Rs...>;
-template <int N, int SIGN, int S, int LS, int NS, int... Rs>
-using StagesLSZ = StagesLSW<N, SIGN, S, LS, 0, true, NS, Rs...>;
-// contiguous sequences (LS = N)
-template <int N, int SIGN, int S, int NS, int... Rs>
-using Stages = StagesLS<N, SIGN, S, N, NS, Rs...>;
 
 }  // namespace wfft
 }  // namespace coral

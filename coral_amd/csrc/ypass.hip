@@ -1,10 +1,9 @@
 // y passes of the horizontal transforms on wavefront-local FFTs.
 //
 // A workgroup owns YL consecutive kx columns of one (variable, z) plane, so
-// every global access covers YL consecutive kx (YL complex = 128 B, 64 B at
-// 768 points) or a whole kept-ky line; each wavefront transforms its own
-// lines in LDS without workgroup barriers (YL/4 of them, one at 768 points
-// and at 384 in FP64).  These are the y-direction parts of c2r_transform
+// every global access covers YL consecutive kx (YL complex = 128 B, 64 B from
+// 486 points) or a whole kept-ky line; each wavefront transforms its own
+// lines in LDS without workgroup barriers (YL / ywaves of them).  These are the y-direction parts of c2r_transform
 // (backward c2c in y) and r2c_transform (forward c2c in y, truncated to the
 // kept ky), slabs.fftw3mpi/transforms.f90:155-301.
 #include "kernels.hpp"
@@ -14,45 +13,61 @@
 
 namespace coral {
 
-using wfft::StagesLSZ;
 using wfft::swz;
 
 
+// Radix plans.  Stages write swizzled where N is a multiple of
+// eight; the other lengths start with a stride-9 or stride-6 stage, whose
+// writes spread over the banks by themselves.  Against the workgroup-level LDS
+// FFT of the other lengths (radices 2 to 4, a barrier per stage), forward and
+// inverse ms per launch: 192^2 x 65 (288 points) 0.29 -> 0.13, 0.13 -> 0.06;
+// 288^2 x 97 (432) 1.08 -> 0.43, 0.54 -> 0.20.
 template <int N>
 struct YPlan;
-template <>
-struct YPlan<96> {
-    template <int SIGN, int S, int LS> using Run = StagesLSZ<96, SIGN, S, LS, 1, 4, 4, 6>;
-};
-template <>
-struct YPlan<144> {
-    template <int SIGN, int S, int LS> using Run = StagesLSZ<144, SIGN, S, LS, 1, 4, 4, 3, 3>;
-};
-template <>
-struct YPlan<192> {
-    template <int SIGN, int S, int LS> using Run = StagesLSZ<192, SIGN, S, LS, 1, 4, 4, 4, 3>;
-};
-template <>
-struct YPlan<384> {
-    template <int SIGN, int S, int LS> using Run = StagesLSZ<384, SIGN, S, LS, 1, 4, 4, 4, 6>;
-};
-template <>
-struct YPlan<768> {
-    template <int SIGN, int S, int LS> using Run = StagesLSZ<768, SIGN, S, LS, 1, 8, 4, 4, 6>;
-};
+#define YPLAN(n, ...)                                                                                        \
+    template <>                                                                                              \
+    struct YPlan<n> {                                                                                        \
+        template <int SIGN, int S, int LS>                                                                   \
+        using Run = wfft::StagesLSW<n, SIGN, S, LS, 0, n % 8 == 0, 1, __VA_ARGS__>;                          \
+    };
+YPLAN(24, 4, 6)
+YPLAN(27, 9, 3)
+YPLAN(36, 6, 6)
+YPLAN(48, 6, 8)
+YPLAN(54, 9, 6)
+YPLAN(72, 9, 8)
+YPLAN(81, 9, 9)
+YPLAN(96, 4, 4, 6)
+YPLAN(108, 9, 12)
+YPLAN(144, 4, 4, 3, 3)
+YPLAN(162, 9, 3, 6)
+YPLAN(192, 4, 4, 4, 3)
+YPLAN(216, 9, 4, 6)
+YPLAN(243, 9, 9, 3)
+YPLAN(288, 9, 4, 8)
+YPLAN(324, 9, 6, 6)
+YPLAN(384, 4, 4, 4, 6)
+YPLAN(432, 9, 6, 8)
+YPLAN(486, 9, 9, 6)
+YPLAN(576, 9, 8, 8)
+YPLAN(648, 9, 9, 8)
+YPLAN(729, 9, 9, 9)
+YPLAN(768, 8, 4, 4, 6)
+#undef YPLAN
 
 // kept ky index jy -> slot of the NYAA-long line
 __device__ inline int ky_slot(int jy, int NY, int N) { return jy < NY / 2 ? jy : N - (NY - 1) + jy; }
 
 // kx columns per workgroup for element type C: one 128-byte segment, 64
-// bytes at 768 points, where a 128-byte tile of lines fills 98 KB of LDS and
-// leaves one workgroup per CU; the 49 KB tile fits three (512^2 x 257: FP64
-// yfwd 5.34 -> 4.61 ms, ybwd 2.30 -> 2.06 ms per launch)
-constexpr int ycol_bytes(int N) { return N == 768 ? 64 : 128; }
+// bytes from 486 points.  At 768 points a 128-byte tile of lines fills 98 KB of
+// LDS and leaves one workgroup per CU; the 49 KB tile fits three (512^2 x 257:
+// FP64 yfwd 5.34 -> 4.61 ms, ybwd 2.30 -> 2.06 ms per launch).
+constexpr int ycol_bytes(int N) { return N >= 486 ? 64 : 128; }
 template <int N, class C>
 constexpr int ycols() { return int(ycol_bytes(N) / sizeof(C)); }
 
-// wavefronts per workgroup.  At 768 points (and 384 in FP64) one line per
+// wavefronts per workgroup.  Two up to 81 points, where four lines still leave
+// lanes idle.  At 768 points (and from 216 in FP64) one line per
 // wavefront rather than four wavefronts of two or four lines each: the
 // tile's LDS bounds the workgroups per CU, so four wavefronts per workgroup
 // left one to three per SIMD, each with two or four lines' butterflies in
@@ -60,7 +75,9 @@ constexpr int ycols() { return int(ycol_bytes(N) / sizeof(C)); }
 // 3.89 -> 3.00 ms per launch).  The FP32 384-point pass measured slower with
 // 16 wavefronts and keeps four.
 template <int N, class C>
-constexpr int ywaves() { return N == 768 || (N == 384 && sizeof(C) == 16) ? ycols<N, C>() : 4; }
+constexpr int ywaves() {
+    return N <= 81 ? 2 : N == 768 || (N >= 216 && sizeof(C) == 16) ? ycols<N, C>() : 4;
+}
 
 // G[b][z][y][ix] = sum_jy Fz[b][z][ix*nky + jy] exp(+i ky y)
 template <int N, class C>
@@ -210,13 +227,20 @@ static bool ypass_wave(hipStream_t st, bool fwd, int N, const C *tw, const C *in
     // otherwise the workgroup-level LDS FFT takes the lines
     if (ywave_lds<C>(N) > lds_limit_current()) return false;
     switch (N) {
-    case 96: go<96>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
-    case 144: go<144>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
-    case 192: go<192>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
-    case 384: go<384>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
-    case 768: go<768>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
-    default: return false;
+#define YCASE(n) \
+    case n: go<n>(st, fwd, tw, in, out, nbatch, NZAA, nkx, nky, NY); return true;
+        YCASE(96) YCASE(144) YCASE(192) YCASE(384) YCASE(768)
+    default: break;
     }
+    if constexpr (std::is_same<C, double2>::value) {   // the FP32 chain keeps to the lengths above
+        switch (N) {
+            YCASE(24) YCASE(27) YCASE(36) YCASE(48) YCASE(54) YCASE(72) YCASE(81) YCASE(108) YCASE(162)
+            YCASE(216) YCASE(243) YCASE(288) YCASE(324) YCASE(432) YCASE(486) YCASE(576) YCASE(648) YCASE(729)
+        default: break;
+        }
+    }
+#undef YCASE
+    return false;
 }
 
 bool launch_ypass_wave(hipStream_t st, bool fwd, const FFTPlan &py, const double2 *in, double2 *out, int nbatch,
