@@ -534,7 +534,7 @@ void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
         std::vector<int2> ucol;
         solve16_ucol(c.stream, Ufull, elem, d.blk_n, bkv, nmat, d.ulen.p, ucol, &d.ustride);
         double lsum = 0.0;
-        for (int j = 0; j < d.blk_n; ++j) lsum += ucol[j].y;
+        for (int j = 0; j < d.blk_n; ++j) lsum += ucol[j + SOLVE16_UPAD].y;
         d.u_mean = lsum / d.blk_n;
         const size_t need = size_t((nmat + 3) / 4) * size_t(d.ustride);
         void *Ut;

@@ -10,6 +10,8 @@
 //   Qhat    [quad][NZ][sys]           Chebyshev coefficients of the products
 #include "kernels.hpp"
 
+#include <type_traits>
+
 #include <cstdio>
 #include <stdexcept>
 
@@ -1319,20 +1321,32 @@ __device__ void split_factors(const T *AB, int n, int kl, int ku, int ldab, T *L
 // solves are interleaved column by column, so that the wavefront's loads of
 // one step fall on adjacent records.  For matrix M (group g = M/4, slot
 // m = M%4), with KLP = solve16_klp(kl):
-//   L:   column j at ((g*ncol16 + j)*4 + m)*KLP: entry k < kl is
-//        L(j + 1 + k, j) (zero for k >= n-1-j and for the padding columns
-//        j >= n);
+//   L:   column j at ((g*ncol16 + j)*4 + m)*KLP, by window slot (below; zero in
+//        the padding columns j >= n);
 //   U:   column j at ((g*nb + j)*4 + m)*(kv+1), nb = 16*ceil(n/16) columns per
 //        matrix (those beyond n stay zero): entry 0 is 1/U(j,j), entry k the
 //        superdiagonal U(j-k, j).
+// Window slots.  The forward sweep keeps the D = solve16_window(kl) rows
+// j .. j+D-1 of step j in lanes ("slots") that never move: no rows are
+// interchanged, the pivot row leaves its slot and the next row of the band
+// takes it.  Which slot holds which row depends on the pivots alone, so it is
+// worked out here, once per factorization: slot[d] is the slot of the row at
+// position j + d (as xGBTF2 interchanges them), lane d of the wavefront.  At
+// column j the pivot (offset p) sits in slot[p], whose number replaces p in
+// piv; the row interchanged with it keeps slot[0].  For kl <= 15 (D = kl + 1)
+// the row at j + D enters the freed slot after the step, with multiplier zero.
+// For kl = 16 (D = 16) the row at j + 16 enters during the step and takes its
+// multiplier there, unless it is the pivot itself (p = 16, kept in piv): then
+// the row at j goes on to position j + 16 in its own slot.
 template <typename T>
-__device__ void split_factors16(const T *AB, int n, int kl, int ku, int ldab, int ncol16, int s, T *L16, T *Ur) {
+__device__ void split_factors16(const T *AB, int n, int kl, int ku, int ldab, int ncol16, int s, T *L16, T *Ur,
+                                unsigned char *piv) {
     using F = Fx<T>;
     const int kv = kl + ku, nb = 16 * ((n + 15) >> 4), g = s >> 2, m = s & 3, klp = solve16_klp(kl);
-    for (int e = threadIdx.x; e < ncol16 * klp; e += blockDim.x) {
-        const int j = e / klp, k = e - j * klp;
-        L16[(((size_t)g * ncol16 + j) * 4 + m) * klp + k] =
-            (j < n && k < min(kl, n - 1 - j)) ? AB[(size_t)j * ldab + kv + 1 + k] : F::zero();
+    const int D = solve16_window(kl), lane = threadIdx.x;
+    for (int e = threadIdx.x; e < (ncol16 - n) * klp; e += blockDim.x) {
+        const int j = n + e / klp, k = e % klp;
+        L16[(((size_t)g * ncol16 + j) * 4 + m) * klp + k] = F::zero();
     }
     for (int e = threadIdx.x; e < n * (kv + 1); e += blockDim.x) {
         int j = e / (kv + 1), k = e % (kv + 1);
@@ -1342,6 +1356,27 @@ __device__ void split_factors16(const T *AB, int n, int kl, int ku, int ldab, in
         else
             v = (j - k >= 0) ? AB[(size_t)j * ldab + kv - k] : F::zero();
         Ur[(((size_t)g * nb + j) * 4 + m) * (kv + 1) + k] = v;
+    }
+    int slot = lane;   // of the row at position j + lane (lanes < D)
+    for (int j0 = 0; j0 < n; j0 += 64) {
+        // 64 columns' pivot offsets in the lanes, one broadcast per column
+        int pl = j0 + lane < n ? piv[j0 + lane] : 0, out = 0;
+        const int cnt = min(64, n - j0);
+        for (int c = 0; c < cnt; ++c) {
+            const int j = j0 + c, p = __builtin_amdgcn_readlane(pl, c);
+            const int first = __builtin_amdgcn_readlane(slot, 0);
+            const int sig = p < D ? __builtin_amdgcn_readlane(slot, p & 63) : p;   // the pivot's slot
+            if (lane == p) slot = first;
+            if (lane == c) out = sig;
+            const int freed = p < D ? sig : first;   // the slot of the row at j + D from the next step on
+            // row j + d (d = 1 .. D): slot[d], the last in the freed slot
+            const int sd = lane == D ? freed : slot;
+            T *rec = L16 + (((size_t)g * ncol16 + j) * 4 + m) * klp;
+            if (lane >= 1 && lane <= D) rec[sd] = (lane <= kl && j + lane < n) ? AB[(size_t)j * ldab + kv + lane] : F::zero();
+            const int nxt = __shfl_down(slot, 1);
+            slot = lane == D - 1 ? freed : nxt;
+        }
+        if (lane < cnt) piv[j0 + lane] = (unsigned char)out;
     }
 }
 
@@ -1405,7 +1440,8 @@ __global__ __launch_bounds__(64) void k_factor(FactorArgs a) {
     T *Lout = REAL ? reinterpret_cast<T *>(a.Lr) : reinterpret_cast<T *>(a.Lf);
     T *Uout = REAL ? reinterpret_cast<T *>(a.Ur) : reinterpret_cast<T *>(a.Uf);
     if (l16)
-        split_factors16<T>(AB, n, kl, ku, ldab, a.ncol16, S, Lout, Uout);
+        split_factors16<T>(AB, n, kl, ku, ldab, a.ncol16, S, Lout, Uout,
+                           a.piv + (size_t)S * 16 * ((n + 15) >> 4));
     else
         split_factors<T>(AB, n, kl, ku, ldab, Lout + (size_t)S * n * kl, Uout + (size_t)S * n * (kv + 1));
 }
@@ -1445,7 +1481,7 @@ __global__ __launch_bounds__(64) void k_factor_lapack16(double2 *work, int n, in
     __syncthreads();
     gbtf2_wave<double2>(AB, n, kl, ku, ldab, piv + (size_t)s * 16 * ((n + 15) >> 4), info + s);
     __syncthreads();
-    split_factors16<double2>(AB, n, kl, ku, ldab, ncol16, s, L16, Ufull);
+    split_factors16<double2>(AB, n, kl, ku, ldab, ncol16, s, L16, Ufull, piv + (size_t)s * 16 * ((n + 15) >> 4));
 }
 
 void launch_factor_lapack16(hipStream_t st, double2 *work, int n, int kl, int ku, int nsys, int ncol16, double2 *L16,
@@ -1689,16 +1725,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 
 // ---------------------------------------------------------------------------
 // Banded solve with four systems per wavefront, sixteen lanes each (kl <= 16).
-// Position 16b + l of a system lives in lane l of its 16-lane row, block b in
-// one register.  Forward (xGBTRS first loop): at step j = 16b + t the row
-// interchange j <-> j + p gathers position j + p with ds_bpermute, the value
-// of position j is broadcast with DPP row_newbcast, and rows j+1 .. j+16 are
-// exactly the 16 lanes (lanes > t in block b, lanes <= t in block b+1), so
-// every lane does useful work.  Backward (xTBSV, column oriented): x_j is
-// broadcast and NQ registers (blocks b .. b-NQ+1) take the column update.
-// Factor records: the interleaved layout of split_factors16, with padding
-// around the U array so that out-of-record reads stay in bounds (their values
-// are masked).
+// Forward (xGBTRS first loop with its row interchanges): the rows a step can
+// touch sit in fixed lanes of the system's 16-lane row (window slots, see
+// split_factors16).  Step j fetches y_j from the pivot's slot with one
+// ds_bpermute (the slot differs per system), puts the band's next row (a DPP
+// row_newbcast of its loaded value) into that slot and takes one
+// multiply-subtract in every lane; lane j mod 16 keeps y_j.  No masks: the
+// freed slot's multiplier is zero, lanes past the window are never read.
+// Interchanging the rows instead took two registers per lane, three selects
+// and two masked updates per step.
+// Backward (xTBSV, column oriented): position 16b + l of a system lives in
+// lane l; x_j is broadcast and NQ registers (blocks b .. b-NQ+1) take the
+// column update; the columns' record offsets and lengths are scalars, loaded a
+// block of 16 at a time, and entries outside a record read as zero through its
+// buffer descriptor.  (With the table in LDS and the bounds in vector
+// registers a step waited for an LDS read and a quarter-rate multiply, and the
+// kernel held 137 VGPRs, now 86.)
+// Small grids are bound by the chain of steps of one wavefront: 64 x 64 x 33
+// 43 -> 31 us per launch, 72 x 48 x 41 54 -> 37, over both sweeps.  From
+// 128^2 x 65 on the launch moves its bytes at 4.0 to 4.4 TB/s, what a device
+// copy reaches, and did not change (256^2 x 129: 1.51 ms).
 // ---------------------------------------------------------------------------
 // row_newbcast writes every lane of the row, so no old value is needed
 template <int T_>
@@ -1736,6 +1782,21 @@ __device__ inline int w_col(unsigned w) { return int((w >> 15) & 0x7FFFu); }
 // windows of consecutive backward steps overlap in cache lines and use
 // ordinary loads, which keep those lines in the cache for the next step.
 //
+// U entries are read through a buffer descriptor of the column's records (a
+// raw buffer: base, byte count), so the hardware's range check returns zero for
+// entries before and past the record; the descriptor is scalar work.
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ inline T buf_load(const T *base, int nelem, unsigned byteoff) {
+    // word 3 of the descriptor: 32-bit data format, no swizzle
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(base), 0, nelem * int(sizeof(T)), 0x00020000);
+    if constexpr (sizeof(T) == 8)
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, byteoff, 0, 0));
+    else
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, byteoff, 0, 0));
+}
+//
 // Scheduling note for the 16-lane solve.  Every value a block starts with
 // (coefficients, right-hand sides, pivots, intermediate results) is loaded
 // one block or PFB steps ahead into a register that the same slot's previous
@@ -1750,84 +1811,71 @@ struct Solve16 {
     // step j's U entries sit in ring slot (j mod 16) mod PFB and are reloaded
     // for step j - PFB, whose slot must be the same
     static_assert(PFB > 0 && 16 % PFB == 0, "the backward prefetch distance must divide 16");
-    // forward step t of a block: swap, eliminate, prefetch the next block's
-    // coefficient.  lo is the lane's position in its row, opaque to the
-    // compiler so that the lane masks are formed where they are used.
-    template <int t>
-    __device__ static inline void fwd_step(double2 &cur, double2 &nxt, const uint4 &pv, T (&ring)[16], const T *Lg,
-                                           unsigned &lcol, int lo, int rowbase, int klp) {
-        const T zero = Fx<T>::zero();
+    // forward step t of a block, then the prefetch of the next block's
+    // coefficient.  cur: the lane's window slot, inc: the rows that enter at
+    // this block's steps, yo collects y.  SEL: kl = 16 (see split_factors16).
+    // lo is the lane's position in its row, opaque to the compiler so that the
+    // lane masks are formed where they are used.
+    template <bool SEL, int t>
+    __device__ static inline void fwd_step(double2 &cur, double2 inc, double2 &yo, const uint4 &pv, T (&ring)[16],
+                                           const T *Lg, unsigned &lrec, int lo, int rowbase, int klp) {
         const unsigned pw = t < 4 ? pv.x : t < 8 ? pv.y : t < 12 ? pv.z : pv.w;
-        const int p = int((pw >> (8 * (t & 3))) & 0xffu);
-        const int tp = t + p;
-        const double2 w = csel(tp < 16, cur, nxt);
-        const double2 bj = bperm_c((rowbase + (tp & 15)) << 2, w);
-        const double2 a = bcast16_c<t>(cur);
-        cur = csel(lo == tp, a, cur);
-        nxt = csel(lo + 16 == tp, a, nxt);
-        cur = csel(lo == t, bj, cur);
-        // lanes whose row is past the band (entry (lo - t - 1) mod 16 >= kl)
-        // loaded the record's last entry and take no update
-        const T c = tsel(unsigned((lo + 15 - t) & 15) < unsigned(klp), ring[t], zero);
-        const bool below = lo > t;
-        cur = submul(cur, tsel(below, c, zero), bj);
-        nxt = submul(nxt, tsel(below, zero, c), bj);
-        asm volatile("" : "+v"(lcol) : "v"(cur.x), "v"(cur.y), "v"(nxt.x), "v"(nxt.y));
-        // entry k = (lo - t - 1) mod 16 of column t of the next block; k >= kl
-        // reads entry kl - 1 (masked at its step)
-        const unsigned kk = min(unsigned((lo + 15 - t) & 15), unsigned(klp - 1));
-        ring[t] = ld_nt(Lg + (size_t)(lcol + kk) + t * 4 * klp);
+        const int sig = int((pw >> (8 * (t & 3))) & 0xffu);
+        const double2 a = bcast16_c<t>(inc);
+        double2 yj = bperm_c((rowbase + (SEL ? sig & 15 : sig)) << 2, cur);
+        if (SEL) yj = csel(sig == 16, a, yj);   // the entering row is the pivot
+        cur = csel(lo == sig, a, cur);
+        cur = submul(cur, ring[t], yj);
+        yo = csel(lo == t, yj, yo);
+        asm volatile("" : "+v"(lrec) : "v"(cur.x), "v"(cur.y));
+        ring[t] = ld_nt(Lg + (size_t)lrec + t * 4 * klp);
         __builtin_amdgcn_sched_barrier(0);   // and not later: the prefetch distance stays 16 steps
     }
 
-    // Lg: the wavefront's multiplier records (uniform); lcol: the offset of
-    // the lane's record of the next block's first column
-    template <int t>
-    __device__ static inline void fwd_block(double2 &cur, double2 &nxt, const uint4 &pv, T (&ring)[16], const T *Lg,
-                                            unsigned &lcol, int lo, int rowbase, int klp) {
-        fwd_step<t>(cur, nxt, pv, ring, Lg, lcol, lo, rowbase, klp);
-        if constexpr (t < 15) fwd_block<t + 1>(cur, nxt, pv, ring, Lg, lcol, lo, rowbase, klp);
+    // Lg: the wavefront's multiplier records (uniform); lrec: the offset of
+    // the lane's entry of the next block's first column
+    template <bool SEL, int t>
+    __device__ static inline void fwd_block(double2 &cur, double2 inc, double2 &yo, const uint4 &pv, T (&ring)[16],
+                                            const T *Lg, unsigned &lrec, int lo, int rowbase, int klp) {
+        fwd_step<SEL, t>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
+        if constexpr (t < 15) fwd_block<SEL, t + 1>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
     }
 
     // backward step t (descending) of a block.  Lane t's q = 0 entry of the
     // ring is record offset 0 of column j, i.e. 1/U(j, j); it is broadcast to
     // the row instead of being loaded separately.  x_j goes to xo.  Entries
-    // outside a column's record were loaded from the group's zeros, so the
-    // updates need no masks; block 0's lanes >= t are finished (their values
-    // live in xo) and may take any update.
-    // Ug: the wavefront's trimmed U records (uniform); ucol: per column (offset
-    // of its four records in the group, record length); m: the lane's matrix
-    // slot.  Entry e = t - lo + 16q of column j is U(j-1-k, j), k = e - 1.
+    // outside a column's record read as zero (buf_load), so the updates need
+    // no masks; block 0's lanes >= t are finished (their values live in xo) and
+    // may take any update.
+    // Ug: the wavefront's trimmed U records (uniform); cn: the records of column
+    // j - PFB, whose entries are fetched here (offset in the group, record
+    // length; length zero before column 0); vm: byte offset of the lane's
+    // matrix and position, (m - 4 lo) entries.  Entry e = t - lo + 16q of
+    // column j is U(j-1-k, j), k = e - 1, at cn.x + 4 e + m.
     template <int t>
-    __device__ static inline void bwd_step(double2 (&r)[NQ], double2 &xo, T (&cring)[PFB][NQ], const T *Ug,
-                                           const int2 *ucol, int m, int lo, int jnext) {
+    __device__ static inline void bwd_step(double2 (&r)[NQ], double2 &xo, T (&cring)[PFB][NQ], const T *Ug, int2 cn,
+                                           unsigned &vm, int lo) {
         constexpr int slot = t % PFB;
         const double2 xj = scale(bcast16_c<t>(r[0]), bcast16<t>(cring[slot][0]));
         xo = csel(lo == t, xj, xo);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) r[q] = submul(r[q], cring[slot][q], xj);
-        // prefetch step jnext = j - PFB (its position in the block: (t - PFB) mod
-        // 16); steps before column 0 are never used and load column 0
+        // prefetch column j - PFB (its position in its block: (t - PFB) mod 16)
         constexpr int tn = (t - PFB) & 15;
-        const int2 cl = ucol[max(jnext, 0)];   // uniform
-        int lb = cl.x + m * cl.y;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(lb) : "v"(r[q].x), "v"(r[q].y));
-        asm volatile("" : "+v"(lb) : "v"(xo.x), "v"(xo.y));
+        for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(vm) : "v"(r[q].x), "v"(r[q].y));
+        asm volatile("" : "+v"(vm) : "v"(xo.x), "v"(xo.y));
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int e = tn + 16 * q - lo;
-            const unsigned off = unsigned(e) < unsigned(cl.y) ? unsigned(lb + e) : 0u;
-            cring[slot][q] = Ug[off];
-        }
+        for (int q = 0; q < NQ; ++q)
+            cring[slot][q] = buf_load(Ug + cn.x, 4 * cn.y, vm + unsigned((tn + 16 * q) * 4 * sizeof(T)));
         __builtin_amdgcn_sched_barrier(0);   // and not later: the prefetch distance stays PFB steps
     }
 
     template <int t>
     __device__ static inline void bwd_block(double2 (&r)[NQ], double2 &xo, T (&cring)[PFB][NQ], const T *Ug,
-                                            const int2 *ucol, int m, int lo, int j0) {
-        bwd_step<t>(r, xo, cring, Ug, ucol, m, lo, j0 + t - PFB);
-        if constexpr (t > 0) bwd_block<t - 1>(r, xo, cring, Ug, ucol, m, lo, j0);
+                                            const int2 (&cl)[16], unsigned &vm, int lo) {
+        bwd_step<t>(r, xo, cring, Ug, cl[t], vm, lo);
+        if constexpr (t > 0) bwd_block<t - 1>(r, xo, cring, Ug, cl, vm, lo);
     }
 };
 
@@ -1838,15 +1886,10 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
     extern __shared__ unsigned sW[];   // position words of every block
     const T *__restrict__ L16 = reinterpret_cast<const T *>(a.L16);
     const T *__restrict__ Ur = reinterpret_cast<const T *>(a.U);
-    const int n = a.n, kv = a.kv, ncol16 = a.ncol16;
+    const int n = a.n, ncol16 = a.ncol16;
     const int lane = threadIdx.x, l = lane & 15, rowbase = lane & 48;
     const int wstride = n + 2 * SOLVE16_WPAD;
     for (int e = lane; e < a.nblk * wstride; e += 64) sW[e] = a.words[e];
-    // U column table after the words (read with uniform addresses in the
-    // backward sweep; in LDS, so that those reads never wait for global loads)
-    const int nbc = 16 * ((n + 15) >> 4);
-    int2 *sU = reinterpret_cast<int2 *>(sW + ((a.nblk * wstride + 1) & ~1));
-    for (int e = lane; e < nbc; e += 64) sU[e] = a.ucol[e];
     // factored matrix (structural block) of this 16-lane row
     const int nmat = a.nsys * a.nblk;
     const int sg = wg * 4 + (lane >> 4);
@@ -1858,7 +1901,8 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
     // x = rhs when its right-hand side is read at the columns too
     const bool idsys = a.ident0 && sys == 0;
     const bool dorot = a.rotate && !idsys;
-    const int g = M >> 2, m = M & 3;
+    // the wavefront's four matrices are one group of records (uniform)
+    const int g = wg, m = M & 3;
     const int klp = solve16_klp(a.kl);
     const T *Lg = L16 + (size_t)g * ncol16 * 4 * klp;   // wavefront's records; matrix m's column j at (4j + m)*klp
     const int B = (n + 15) >> 4;
@@ -1885,40 +1929,55 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
     };
 
     // ---- forward ----
-    {
-        const unsigned w0 = W[l], w1 = W[16 + l];
-        double2 cur = fix_rhs(b[row_or0(w0)], w0), nxt = fix_rhs(b[row_or0(w1)], w1);
+    auto forward = [&](auto sel) {
+        constexpr bool SEL = decltype(sel)::value;
+        const int D = solve16_window(a.kl);   // rows in the window; row D + 16 b + l enters at step l of block b
+        const unsigned w0 = W[l], w1 = W[D + l];
+        double2 cur = csel(l < D, fix_rhs(b[row_or0(w0)], w0), make_double2(0.0, 0.0)), yo = make_double2(0.0, 0.0);
+        double2 inc = fix_rhs(b[row_or0(w1)], w1);
         uint4 pv = P[0];
         T ring[16];
-        const unsigned lbase = unsigned(m * klp);
+        // the lane's entry of a record (lanes past the window read the last one)
+        const unsigned lbase = unsigned(m * klp + min(l, klp - 1));
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
-            const unsigned kk = min(unsigned((l + 15 - t) & 15), unsigned(klp - 1));
-            ring[t] = ld_nt(Lg + lbase + kk + t * 4 * klp);
+            ring[t] = ld_nt(Lg + lbase + t * 4 * klp);
             __builtin_amdgcn_sched_barrier(0);   // in the order of use
         }
         for (int bk = 0; bk < B; ++bk) {
             int lo = l;
             asm volatile("" : "+v"(lo));
-            // loaded here, consumed at the end of this block: the right-hand
-            // side of block bk+2 and the pivots of block bk+1
-            const unsigned w2 = W[bk * 16 + 32 + l];
+            // loaded here, consumed at the end of this block: the rows that
+            // enter in block bk+1 and its pivots
+            const unsigned w2 = W[bk * 16 + 16 + D + l];
             const double2 nx2 = b[row_or0(w2)];
             const uint4 pvn = P[min(bk + 1, B - 1)];
-            unsigned lcol = lbase + unsigned(bk * 16 + 16) * unsigned(4 * klp);
-            S::template fwd_block<0>(cur, nxt, pv, ring, Lg, lcol, lo, rowbase, klp);
-            *out_ptr(W[bk * 16 + l]) = cur;   // intermediate, kept at the unknown's slot
-            cur = nxt;
-            nxt = fix_rhs(nx2, w2);
+            unsigned lrec = lbase + unsigned(bk * 16 + 16) * unsigned(4 * klp);
+            S::template fwd_block<SEL, 0>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
+            *out_ptr(W[bk * 16 + l]) = yo;   // intermediate, kept at the unknown's slot
+            inc = fix_rhs(nx2, w2);
             pv = pvn;
         }
-    }
+    };
+    if (a.kl < 16)
+        forward(std::false_type{});
+    else
+        forward(std::true_type{});
     __threadfence_block();
 
     // ---- backward ----
     // trimmed U records of the wavefront's group (see Solve16Args::U)
     const T *Ug = Ur + (size_t)g * a.ustride;
-    const int2 *ucol = sU;
+    // per column the offset of its records in the group and their length, from
+    // column -SOLVE16_UPAD on; read as scalars, a block's 16 at its start
+    static_assert(PFB == SOLVE16_UPAD, "the column table is padded for the prefetch distance");
+    // (through the constant address space: nothing here writes the table)
+    typedef const __attribute__((address_space(4))) unsigned long long *CWords;
+    const CWords ucol = (CWords)(uintptr_t)a.ucol;
+    auto column = [&](int k) -> int2 {
+        const unsigned long long w = ucol[k];
+        return make_int2(int(unsigned(w)), int(unsigned(w >> 32)));
+    };
     double2 r[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -1926,17 +1985,14 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
         r[q] = fix_y(y[col_or0(wq)], wq);
     }
     T cring[PFB][NQ];
+    const unsigned vm0 = unsigned((m - 4 * l) * int(sizeof(T)));
 #pragma unroll
     for (int u = 0; u < PFB; ++u) {
         // step j = 16B - 1 - u lives in slot (15 - u) % PFB
-        const int j = B * 16 - 1 - u;
-        const int t = j & 15;
-        const int2 cl = ucol[j];
+        const int2 cn = column(B * 16 - 1 - u + SOLVE16_UPAD);
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int e = t + 16 * q - l;
-            cring[(15 - u) % PFB][q] = Ug[unsigned(e) < unsigned(cl.y) ? unsigned(cl.x + m * cl.y + e) : 0u];
-        }
+        for (int q = 0; q < NQ; ++q)
+            cring[(15 - u) % PFB][q] = buf_load(Ug + cn.x, 4 * cn.y, vm0 + unsigned((15 - u + 16 * q) * 4 * sizeof(T)));
         // issued in the order of use: the loop's first wait then counts the
         // same way whether it is entered from here or from its own end
         __builtin_amdgcn_sched_barrier(0);
@@ -1949,7 +2005,12 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
         // block bk-NQ, which enters the window of blocks being updated
         const unsigned wy = W[(bk - NQ) * 16 + l];
         const double2 ynx = y[col_or0(wy)];
-        S::template bwd_block<15>(r, xo, cring, Ug, ucol, m, lo, bk * 16);
+        // columns 16 bk - PFB .. 16 bk + 15 - PFB, fetched during this block
+        int2 cl[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) cl[t] = column(bk * 16 + t);
+        unsigned vm = vm0;
+        S::template bwd_block<15>(r, xo, cring, Ug, cl, vm, lo);
         const unsigned w0 = W[bk * 16 + l];
         *out_ptr(w0) = rot_out(xo, code(w0));
 #pragma unroll
@@ -1981,8 +2042,7 @@ static bool launch_solve16(hipStream_t st, const Solve16Args &a) {
     if (a.kl > 16 || a.n < 32 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol) return false;
     const int nq = 1 + (a.kv + 15) / 16;
     const dim3 grid((a.nsys * a.nblk + 3) / 4);
-    const size_t lds = (size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) + 1) / 2 * 2 * sizeof(unsigned) +
-                       size_t(16 * ((a.n + 15) / 16)) * sizeof(int2);
+    const size_t lds = size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) * sizeof(unsigned);
     if (lds > 32768 || !a.sink) return false;
     switch (nq) {
     case 2: hipLaunchKernelGGL((k_solve16<T, 2, 8>), grid, dim3(64), lds, st, a); break;
@@ -2036,9 +2096,9 @@ __global__ void k_u_trim(const T *__restrict__ U, int n, int kv, int nmat, const
     if (idx >= (long long)nmat * nb) return;
     const int M = int(idx / nb), j = int(idx % nb), g = M >> 2, m = M & 3;
     const T *rec = U + ((size_t)(g * nb + j) * 4 + m) * (kv + 1);
-    const int2 cl = ucol[j];
-    T *out = Ut + (size_t)g * ustride + cl.x + m * cl.y;
-    for (int e = 0; e < cl.y; ++e) out[e] = rec[e];
+    const int2 cl = ucol[j + SOLVE16_UPAD];
+    T *out = Ut + (size_t)g * ustride + cl.x + m;
+    for (int e = 0; e < cl.y; ++e) out[4 * e] = rec[e];
 }
 
 void solve16_ucol(hipStream_t st, const void *Ufull, int elem, int n, int kv, int nmat, int *scratch_len,
@@ -2058,10 +2118,10 @@ void solve16_ucol(hipStream_t st, const void *Ufull, int elem, int n, int kv, in
     if (hipMemcpyAsync(len.data(), scratch_len, nb * sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         throw std::runtime_error("download of U column lengths failed");
-    ucol.assign(nb, make_int2(0, 0));
-    long long off = 16;   // [0, 16) of every group stays zero
+    ucol.assign(nb + SOLVE16_UPAD, make_int2(0, 0));
+    long long off = 0;
     for (int j = 0; j < nb; ++j) {
-        ucol[j] = make_int2(int(off), len[j]);
+        ucol[j + SOLVE16_UPAD] = make_int2(int(off), len[j]);
         off += 4LL * len[j];
     }
     *ustride = off;
@@ -2091,8 +2151,7 @@ bool solve16_shape(const Solve16Args &a, int &nwg, size_t &lds, int &nq) {
     nq = 1 + (a.kv + 15) / 16;
     if (nq < 2 || nq > 4) return false;
     nwg = (a.nsys * a.nblk + 3) / 4;
-    lds = (size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) + 1) / 2 * 2 * sizeof(unsigned) +
-          size_t(16 * ((a.n + 15) / 16)) * sizeof(int2);
+    lds = size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) * sizeof(unsigned);
     return lds <= 32768;
 }
 

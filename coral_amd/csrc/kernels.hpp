@@ -286,26 +286,30 @@ void launch_solve(hipStream_t st, const double2 *Lf, const double2 *Uf, const un
 // 16-lane solve (four systems per wavefront): columns per system of its
 // multiplier records, or 0 when the band does not fit (kl > 16, kv > 47)
 int solve16_ncol(int n, int kl, int kv);
-// entries per multiplier record of the 16-lane solve: the kl multipliers of a
-// column (at least one entry)
-__host__ __device__ inline int solve16_klp(int kl) { return kl < 1 ? 1 : kl; }
+// rows in the window of the 16-lane solve's forward sweep (see split_factors16
+// in kernels.hip), and the entries per multiplier record, one per window slot
+__host__ __device__ inline int solve16_window(int kl) { return kl < 16 ? kl + 1 : 16; }
+__host__ __device__ inline int solve16_klp(int kl) { return solve16_window(kl); }
 // U arrays of the solves carry this many elements of padding on each side (the
 // 16-lane solve reads up to 16 elements before the first record and 64 past
 // the last)
 constexpr int SOLVE16_PAD = 2048;
+// columns before the first in the solve's table of trimmed U records: the
+// backward sweep fetches that many steps ahead
+constexpr int SOLVE16_UPAD = 8;
 // 16-lane solve of nsys systems of `total` unknowns, each made of nblk
 // structural blocks of n unknowns and band (kl, kv - kl) (see FactorArgs);
 // factors in the layout k_factor writes for ncol16 > 0.
 struct Solve16Args {
     const void *L16;             // double (real form) or double2
-    // U records trimmed per column (solve16_trim_u): for wavefront group g,
-    // column j, matrix slot m and entry e < len_j at U + g*ustride + cb_j +
-    // m*len_j + e, with ucol[j] = (cb_j, len_j); U + g*ustride + [0, 16) is zero
+    // U records trimmed per column (solve16_trim_u_copy): for wavefront group
+    // g, column j, matrix slot m and entry e < len_j at U + g*ustride + cb_j +
+    // 4*e + m, with ucol[j + SOLVE16_UPAD] = (cb_j, len_j)
     const void *U;
     const int2 *ucol;
     long long ustride;
     int ncol16;
-    const unsigned char *piv;    // [nsys*nblk][16*ceil(n/16)], zero past n
+    const unsigned char *piv;    // [nsys*nblk][16*ceil(n/16)] window slots of the pivots, zero past n
     // position words (solve16_words): row and column of the system at each
     // position of a block, and their real-form rotations
     const unsigned *words;
@@ -319,8 +323,9 @@ struct Solve16Args {
 // Trimmed U records of the 16-lane layout: the full records of kv+1 entries
 // at Ufull (as k_factor writes them, nmat matrices of n unknowns, elem bytes
 // per entry) are cut to the longest nonzero prefix each column has in any
-// matrix.  solve16_ucol fills ucol (16*ceil(n/16) columns: offset of the
-// column's four records in a group, record length) and the group stride
+// matrix.  solve16_ucol fills ucol (SOLVE16_UPAD empty records, then
+// 16*ceil(n/16) columns: offset of the column's four records in a group, record
+// length) and the group stride
 // (scratch_len: that many ints of device memory); solve16_trim_u_copy then
 // repacks into Utrim (ngroups * ustride elements, cleared by the caller).
 void solve16_ucol(hipStream_t st, const void *Ufull, int elem, int n, int kv, int nmat, int *scratch_len,
