@@ -61,8 +61,10 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def solve_bytes(N, nsys, real, blocks, u_entries):
-    """Algorithmic HBM bytes of one banded-solve launch.  Each system is factored
+def solve_bytes(N, nsys, real, blocks, u_entries, nfactored=None):
+    """Algorithmic HBM bytes of one banded-solve launch.  Each of nfactored
+    systems (all nsys of them unless symmetries let related wavenumbers share
+    one factorization) is factored
     as nblk structural blocks of blk_n unknowns with band (bl, bu): per column
     bl multipliers, u_entries U entries (the mean length of the U records,
     each cut to the longest nonzero prefix its column has over all
@@ -72,7 +74,8 @@ def solve_bytes(N, nsys, real, blocks, u_entries):
     all systems and not counted.)"""
     nblk, blk_n, bl, bu = blocks
     e = 8 if real else 16
-    return int(nsys * (nblk * blk_n * (e * bl + e * u_entries + 1) + N * (16 + 16)))
+    nfac = nsys if nfactored is None else nfactored
+    return int(nfac * nblk * blk_n * (e * bl + e * u_entries + 1) + nsys * N * (16 + 16))
 
 
 def kernel_bytes(name, P):
@@ -81,7 +84,7 @@ def kernel_bytes(name, P):
     nf, nq = P["nfull"], P["nquad"]
     S_sys = 16 * N * nsys
     table = {
-        "solve": solve_bytes(N, nsys, P["real"], P["blocks"], P["u_entries"]),
+        "solve": solve_bytes(N, nsys, P["real"], P["blocks"], P["u_entries"], P.get("nfactored")),
         # M (a x^n + b x_1) + K_hat terms: ARS_222 reads 2 (stage 1) and 4 (stage 2)
         # state vectors and writes one, 4 on average per launch
         "rhs": 4 * S_sys,
@@ -642,7 +645,7 @@ def main():
         log(f"value check: 20 steps at amplitude 1e-2 {vc[1e-2][0]:.3f} ms/step, at {amp:g} {vc[amp][0]:.3f} ms/step")
 
     P = dict(N=total, kl=kl, ku=ku, nsys=nsys, real=g.factor_is_real(0), blocks=g.factor_blocks(0),
-             u_entries=g.u_entries_per_column(0), NZ=NZ,
+             u_entries=g.u_entries_per_column(0), nfactored=g.factored_systems(0)[0], NZ=NZ,
              NZAA=3 * NZ // 2, NYAA=3 * NX // 2, nkx=NX // 2,
              nfull=len(recipe.full_vars), nquad=len(recipe.quad_vars))
     per_kernel = {}

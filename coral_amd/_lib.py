@@ -70,7 +70,8 @@ EXPORTS = (
     "coral_amd_bwd_transform", "coral_amd_fwd_transform", "coral_amd_banded_solve",
     "coral_amd_timers_enable", "coral_amd_timer_read", "coral_amd_assembled_operator", "coral_amd_use_graphs", "coral_amd_products",
     "coral_amd_factor_kind", "coral_amd_get_variable_physical", "coral_amd_set_variable_physical",
-    "coral_amd_horizontal_averages", "coral_amd_factor_blocks", "coral_amd_system_solve",
+    "coral_amd_horizontal_averages", "coral_amd_factor_blocks", "coral_amd_factored_systems",
+    "coral_amd_system_solve",
     "coral_amd_set_precision", "coral_amd_set_kx0_projection", "coral_amd_banded_solve_noalloc",
     "coral_amd_banded_solve_noalloc_bytes", "coral_amd_set_launch_shape", "coral_amd_get_launch_shape",
     "coral_amd_ensemble_create", "coral_amd_ensemble_destroy", "coral_amd_ensemble_set_schedule",
@@ -106,6 +107,7 @@ def _load():
     lib.coral_amd_wavenumbers.argtypes = [P, P, P, P, P]
     lib.coral_amd_system_info.argtypes = [P, c_int32, P, P, P, P]
     lib.coral_amd_factor_blocks.argtypes = [P, c_int32, c_int32, P, P, P, P, P]
+    lib.coral_amd_factored_systems.argtypes = [P, c_int32, P, P]
     lib.coral_amd_bwd_transform.argtypes = [P, P, P]
     lib.coral_amd_fwd_transform.argtypes = [P, P, P]
     lib.coral_amd_system_solve.argtypes = [P, c_int32, P, P]

@@ -10,6 +10,8 @@
 //   NL insertion            PL_IMEX_timestepping_marching.f90:306-350
 #include "assembly.hpp"
 
+#include <functional>
+#include <array>
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -234,6 +236,102 @@ static void find_real_form(const coral_amd_system &s, SystemTables &t) {
         for (int c = 0; c < t.var_size[v]; ++c) var_at[t.posP[t.var_first[v] + c]] = v;
     for (int p = 0; p < t.total; ++p)
         t.rot[p] = (unsigned char)(val[t.pos_eqn[p]] | (val[nv + var_at[p]] << 1));
+}
+
+// A symmetry of the operators (see SystemTables::Symmetry).  At k' a piece
+// (i kx)^a (i ky)^b becomes (-1)^b times itself (reflection), or (-1)^b
+// (i kx)^b (i ky)^a (rotation).  The search runs over the involutions of the
+// variables (swapping only variables of one boundary-condition code) and of
+// the equations (of one order); for each, the signs are a two-colouring of the
+// graph (equation, variable) whose edges are the pieces, which must map onto
+// pieces of equal magnitude.
+static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotate, SystemTables::Symmetry &sym) {
+    const int nv = s.nvars;
+    if (nv > 8) return;   // 764 involutions each at 8
+    // coefficients by (mass or stiffness, equation, variable, iz, mz, a, b)
+    std::map<std::array<int, 7>, double> c;
+    for (int k = 0; k < s.n_mass + s.n_stif; ++k) {
+        const coral_amd_piece &p = k < s.n_mass ? s.mass[k] : s.stif[k - s.n_mass];
+        if (p.dsca != 0.0) c[{k < s.n_mass ? 0 : 1, p.eqn, p.var, p.iz, p.mz, p.kx, p.ky}] += p.dsca;
+    }
+    auto involutions = [nv](const int32_t *kind) {
+        std::vector<std::vector<int>> out;
+        std::vector<int> cur(nv, -1);
+        std::function<void(int)> go = [&](int i) {
+            while (i < nv && cur[i] >= 0) ++i;
+            if (i == nv) {
+                out.push_back(cur);
+                return;
+            }
+            for (int j = i; j < nv; ++j) {
+                if (cur[j] >= 0 || kind[i] != kind[j]) continue;
+                cur[i] = j;
+                cur[j] = i;
+                go(i + 1);
+                cur[i] = cur[j] = -1;
+            }
+        };
+        go(0);
+        return out;
+    };
+    const auto vars = involutions(s.bc_codes), eqns = involutions(s.eqn_orders);
+    for (const auto &pe : eqns)
+        for (const auto &pv : vars) {
+            // edges (equation of k', variable of k', parity of the sign), checked for magnitude
+            bool ok = true;
+            std::vector<std::vector<std::pair<int, int>>> adj(2 * nv);
+            for (const auto &[key, val] : c) {
+                const auto [op, e, v, iz, mz, a, b] = key;   // at k' : (e, v)
+                const auto it = c.find({op, pe[e], pv[v], iz, mz, rotate ? b : a, rotate ? a : b});
+                if (it == c.end() || std::fabs(it->second) != std::fabs(val)) {
+                    ok = false;
+                    break;
+                }
+                const int par = ((b & 1) != 0) ^ ((it->second < 0) != (val < 0));
+                adj[e].push_back({nv + v, par});
+                adj[nv + v].push_back({e, par});
+            }
+            if (!ok) continue;
+            std::vector<int> neg(2 * nv, -1);
+            for (int root = 0; root < 2 * nv && ok; ++root) {
+                if (neg[root] >= 0) continue;
+                neg[root] = 0;
+                std::vector<int> stack{root};
+                while (!stack.empty() && ok) {
+                    const int u = stack.back();
+                    stack.pop_back();
+                    for (auto [w, par] : adj[u]) {
+                        if (neg[w] < 0) {
+                            neg[w] = neg[u] ^ par;
+                            stack.push_back(w);
+                        } else if (neg[w] != (neg[u] ^ par)) {
+                            ok = false;
+                            break;
+                        }
+                    }
+                }
+            }
+            if (!ok) continue;
+            sym.found = true;
+            sym.row.assign(t.total, 0);
+            sym.col.assign(t.total, 0);
+            sym.rneg.assign(t.total, 0);
+            sym.cneg.assign(t.total, 0);
+            for (int i = 0; i < nv; ++i) {
+                // (pe and pv are their own inverses)
+                for (int r = 0; r < t.eqn_size[i]; ++r) {
+                    const int at = t.posQ[t.eqn_first[i] + r];
+                    sym.row[at] = t.posQ[t.eqn_first[pe[i]] + r];
+                    sym.rneg[at] = (unsigned char)neg[pe[i]];
+                }
+                for (int r = 0; r < t.var_size[i]; ++r) {
+                    const int at = t.posP[t.var_first[i] + r];
+                    sym.col[at] = t.posP[t.var_first[pv[i]] + r];
+                    sym.cneg[at] = (unsigned char)neg[nv + pv[i]];
+                }
+            }
+            return;
+        }
 }
 
 // Structural blocks (see SystemTables::nblk): union-find over rows (0..n-1)
@@ -503,6 +601,10 @@ static SystemTables build_system(const coral_amd_system &s, int NZ, double cente
     for (int e = 0; e < s.nvars; ++e) t.nl_eqn_begin[e + 1] += t.nl_eqn_begin[e];
     find_real_form(s, t);
     find_blocks(t);
+    if (kxky) {
+        find_symmetry(s, t, false, t.reflect);
+        find_symmetry(s, t, true, t.rotate);
+    }
     return t;
 }
 

@@ -83,6 +83,17 @@ struct SystemTables {
     int nblk = 1, nblk_n = 0, blk_nl = 0, blk_nu = 0;
     std::vector<int> blk_row, blk_col;   // [nblk][nblk_n]
     int band_width() const { return nl + nu + 1; }
+    // Symmetries of the operators between wavenumbers: where they exist, the
+    // system at k' = (kx, -ky) (SYM_REFLECT) or k' = (ky, -kx) (SYM_ROTATE, for
+    // equal box lengths) is that at k with rows and columns renumbered and some
+    // signs changed: A(k')(row[i], col[j]) = rsign[i] csign[j] A(k)(i, j) for M and
+    // L alike, so one factorization serves both wavenumbers.
+    struct Symmetry {
+        bool found = false;
+        std::vector<int> row, col;                 // position at k -> position at k'
+        std::vector<unsigned char> rneg, cneg;     // 1: sign -1
+    };
+    Symmetry reflect, rotate;
 };
 
 // Extraction of a full-variable term: Chebyshev coefficient n of the term is

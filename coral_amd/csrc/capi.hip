@@ -2,9 +2,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -70,7 +72,13 @@ struct SysDev {
     // (SystemTables::nblk; 1 = the whole system)
     int nblk = 1, blk_n = 0, blk_nl = 0, blk_nu = 0;
     DevBuf<int> blk_row, blk_col;
-    DevBuf<unsigned> words;      // position words of the 16-lane solve (solve16_words)
+    // position words of the 16-lane solve (solve16_words), one table per slot
+    DevBuf<unsigned> words;
+    // systems factored and the systems each serves (Solve16Args::mem): all of
+    // them, or one of each set that the operators' symmetries relate
+    int nrep = 0, nslot = 1;
+    std::vector<int> rep_h;
+    DevBuf<int> rep, mem;
     // trimmed U records of the 16-lane solve (solve16_ucol), rebuilt at every
     // factorization
     DevBuf<double> Urt;
@@ -325,6 +333,74 @@ FFTPlan make_plan(int N, DevBuf<double2> &tw) {
     return p;
 }
 
+// Which wavenumbers share factors (SystemTables::Symmetry): d.rep_h the systems
+// factored, d.mem the systems each serves, syms the symmetry of slots 1 .. .
+// With the reflection, (kx, ky) and (kx, -ky) share; with the rotation, (kx, ky)
+// and (ky, -kx), which needs equal box lengths; with both, those four and
+// (ky, kx).  Factors are two thirds of what a solve reads.  The (0, 0) system is
+// the identity and stands alone.  CORAL_AMD_NO_SHARED_FACTORS=1 before
+// coral_amd_create factors every system.
+void share_factors(SysDev &d, const KeptModes &km, std::vector<Solve16Sym> &syms) {
+    const SystemTables &t = *d.t;
+    const char *off = std::getenv("CORAL_AMD_NO_SHARED_FACTORS");
+    if (off && off[0] == '1') return;
+    const bool refl = t.reflect.found, rota = t.rotate.found && km.kx_box == km.ky_box;
+    if (!refl && !rota) return;
+    auto as_sym = [](const SystemTables::Symmetry &y) { return Solve16Sym{y.row, y.col, y.rneg, y.cneg}; };
+    const int nslot = refl && rota ? 4 : 2;
+    // (two right-hand sides' word tables fit the solve's LDS)
+    if (2 * size_t(d.nblk) * (d.blk_n + 2 * SOLVE16_WPAD) * sizeof(unsigned) > 32768) return;
+    typedef std::pair<int, int> K;
+    const std::function<K(K)> F = [](K k) { return K(k.first, -k.second); }, R = [](K k) { return K(k.second, -k.first); };
+    std::vector<std::function<K(K)>> ops;
+    if (refl) {
+        ops.push_back(F);
+        syms.push_back(as_sym(t.reflect));
+    }
+    if (rota) {
+        ops.push_back(R);
+        syms.push_back(as_sym(t.rotate));
+    }
+    if (nslot == 4) {
+        // the reflection after the rotation: (ky, kx)
+        ops.push_back([&](K k) { return F(R(k)); });
+        Solve16Sym c = as_sym(t.rotate);
+        for (int i = 0; i < t.total; ++i) {
+            c.rneg[i] ^= t.reflect.rneg[c.row[i]];
+            c.cneg[i] ^= t.reflect.cneg[c.col[i]];
+            c.row[i] = t.reflect.row[c.row[i]];
+            c.col[i] = t.reflect.col[c.col[i]];
+        }
+        syms.push_back(c);
+    }
+    auto index = [&](K k) -> int {
+        if (k.first < 0 || k.first >= km.nkx || std::abs(k.second) >= km.NY / 2) return -1;
+        return k.first * km.nky + (k.second >= 0 ? k.second : k.second + km.NY - 1);
+    };
+    std::vector<char> done(d.nsys, 0);
+    std::vector<int> mem;
+    for (int pass = 0; pass < 2; ++pass)   // first the wavenumbers whose partners are all kept
+        for (int kx = 0; kx < km.nkx; ++kx)
+            for (int ky = -(km.NY / 2 - 1); ky < km.NY / 2; ++ky) {
+                const K k(kx, ky);
+                const int s = index(k);
+                if (done[s] || (pass == 0 && (kx == 0 || ky < 0))) continue;
+                done[s] = 1;
+                d.rep_h.push_back(s);
+                mem.push_back(s);
+                for (int q = 1; q < nslot; ++q) {
+                    const int o = kx == 0 && ky == 0 ? -1 : index(ops[q - 1](k));
+                    const bool take = o >= 0 && !done[o];
+                    if (take) done[o] = 1;
+                    mem.push_back(take ? o : -1);
+                }
+            }
+    d.nslot = nslot;
+    d.nrep = int(d.rep_h.size());
+    d.rep.upload(d.rep_h);
+    d.mem.upload(mem);
+}
+
 void fill_system_device(SysDev &d, int nstages, const KeptModes &km, hipStream_t st, int NZ) {
     SystemTables &t = *d.t;
     const size_t n = size_t(d.nsys) * t.total;
@@ -457,11 +533,21 @@ void fill_system_device(SysDev &d, int nstages, const KeptModes &km, hipStream_t
         d.blk_nl = t.nl;
         d.blk_nu = t.nu;
     }
-    if (d.ncol16 > 0)
-        d.words.upload(solve16_words(t.total, d.nblk, d.blk_n, split ? t.blk_row.data() : nullptr,
-                                     split ? t.blk_col.data() : nullptr, d.real ? t.rot.data() : nullptr));
+    d.nrep = d.nsys;
+    if (d.ncol16 > 0) {
+        std::vector<Solve16Sym> syms;
+        if (d.kxky) share_factors(d, km, syms);
+        std::vector<unsigned> words;
+        for (int k = 0; k < d.nslot; ++k) {
+            const auto w = solve16_words(t.total, d.nblk, d.blk_n, split ? t.blk_row.data() : nullptr,
+                                         split ? t.blk_col.data() : nullptr, d.real ? t.rot.data() : nullptr,
+                                         k ? &syms[k - 1] : nullptr);
+            words.insert(words.end(), w.begin(), w.end());
+        }
+        d.words.upload(words);
+    }
     const int bkv = d.blk_nl + d.blk_nu;
-    const size_t nmat = size_t(d.nsys) * d.nblk, nmat4 = (nmat + 3) / 4 * 4;
+    const size_t nmat = size_t(d.nrep) * d.nblk, nmat4 = (nmat + 3) / 4 * 4;
     const size_t nb = 16 * ((size_t(d.blk_n) + 15) / 16);
     const size_t lsize = d.ncol16 > 0 ? nmat4 * d.ncol16 * solve16_klp(d.blk_nl)
                                       : size_t(d.nsys) * t.total * std::max(t.nl, 1);
@@ -490,8 +576,8 @@ void fill_zero(hipStream_t st, double2 *p, size_t n);
 
 void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
     SystemTables &t = *d.t;
-    // matrices factored: nblk structural blocks of blk_n unknowns per system
-    const int nmat = d.nsys * d.nblk, ldab = 2 * d.blk_nl + d.blk_nu + 1;
+    // matrices factored: nblk structural blocks of blk_n unknowns per factored system
+    const int nmat = d.nrep * d.nblk, ldab = 2 * d.blk_nl + d.blk_nu + 1;
     const size_t per = size_t(d.blk_n) * ldab;
     // bound the working band to ~1 GiB per launch
     int chunk = int(std::max<size_t>(1, (size_t(1) << 30) / (per * sizeof(double2))));
@@ -525,6 +611,7 @@ void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
         a.blk_col = d.blk_col.p;
         a.piv = d.piv.p;
         a.info = d.info.p;
+        a.rep = d.rep.p;
         c.timed("factor", [&] { launch_factor(c.stream, a); });
     }
     if (d.ncol16 > 0) {
@@ -556,7 +643,8 @@ void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
         if (info[m] != 0)
             throw std::runtime_error("singular evolution operator (zgbtrf info " + std::to_string(info[m]) +
                                      (d.nblk > 1 ? " in structural block " + std::to_string(m % d.nblk) : "") +
-                                     ") at wavenumber index " + std::to_string(m / d.nblk));
+                                     ") at wavenumber index " +
+                                     std::to_string(d.rep_h.empty() ? m / d.nblk : d.rep_h[m / d.nblk]));
 }
 
 // y = M (sum ma U) + L (sum xa X) + sum kb K
@@ -1428,13 +1516,15 @@ bool solve16_args_of(const coral_amd_ctx &c, const SysDev &d, const double2 *rhs
     sa.ncol16 = d.ncol16;
     sa.piv = d.piv.p;
     sa.words = d.words.p;
+    sa.mem = d.mem.p;
+    sa.nslot = d.nslot;
     sa.rotate = d.real ? 1 : 0;
     sa.ident0 = d.kxky ? 1 : 0;
     sa.total = t.total;
     sa.n = d.blk_n;
     sa.kl = d.blk_nl;
     sa.kv = d.blk_nl + d.blk_nu;
-    sa.nsys = d.nsys;
+    sa.nsys = d.nrep;
     sa.nblk = d.nblk;
     sa.rhs = rhs;
     sa.x = out;
@@ -2017,6 +2107,16 @@ int coral_amd_factor_kind(coral_amd_ctx *c, int32_t isys, int32_t *is_real) {
     }
 }
 
+int coral_amd_factored_systems(coral_amd_ctx *c, int32_t isys, int32_t *nfactored, int32_t *nshare) {
+    if (!c || isys < 0 || isys >= int(c->ks.size())) {
+        g_err = "system index out of range";
+        return -1;
+    }
+    if (nfactored) *nfactored = c->ks[isys]->nrep;
+    if (nshare) *nshare = c->ks[isys]->nslot;
+    return 0;
+}
+
 int coral_amd_factor_blocks(coral_amd_ctx *c, int32_t kind, int32_t isys, int32_t *nblk, int32_t *blk_n,
                             int32_t *blk_nl, int32_t *blk_nu, double *u_entries) {
     try {
@@ -2465,6 +2565,7 @@ int coral_amd_banded_solve(int32_t device, int32_t n, int32_t kl, int32_t ku, in
             sa.ncol16 = ncol16;
             sa.piv = piv.p;
             sa.words = words.p;
+            sa.nslot = 1;
             sa.rotate = 0;
             sa.ident0 = 0;
             sa.total = n;
@@ -3263,7 +3364,7 @@ void ens_capture_lockstep(coral_amd_ensemble &e) {
     const int s = e.runs[0]->P.nstages;
     size_t nks = 0;
     for (auto *c : e.runs) nks += c->ks.size();
-    const size_t cap_args = 2 * size_t(s) * std::max<size_t>(nks, 1), cap_start = 2 * size_t(s) * (nks + 8);
+    const size_t cap_args = 2 * size_t(s) * std::max<size_t>(nks, 1), cap_start = 2 * size_t(s) * (2 * nks + 1);
     e.lk_args_h.assign(cap_args, Solve16Args{});
     e.lk_start_h.assign(cap_start, 0);
     e.lk_args.alloc(cap_args);
@@ -3304,19 +3405,20 @@ void ens_capture_lockstep(coral_amd_ensemble &e) {
                     }
                 }
                 for (auto *c : e.runs) c->stream = st;
-                // (real form, NQ) -> the group's arguments, workgroups and LDS
-                std::map<std::pair<int, int>, std::vector<std::pair<Solve16Args, int>>> groups;
-                std::map<std::pair<int, int>, size_t> glds;
+                // (real form, NQ, NR) -> the group's arguments, workgroups and LDS
+                std::map<std::array<int, 3>, std::vector<std::pair<Solve16Args, int>>> groups;
+                std::map<std::array<int, 3>, Solve16Shape> gshape;
                 for (auto *c : e.runs)
                     for (auto &d : c->ks) {
                         Solve16Args sa;
-                        int nwg = 0, nq = 0;
-                        size_t lds = 0;
-                        if (solve16_args_of(*c, *d, d->R.p, d->X[i]->p, sa) && solve16_shape(sa, nwg, lds, nq)) {
+                        Solve16Shape sh;
+                        if (solve16_args_of(*c, *d, d->R.p, d->X[i]->p, sa) && solve16_shape(sa, sh)) {
                             if (!d->real) sa.rotate = 0;
-                            const auto key = std::make_pair(d->real ? 1 : 0, nq);
-                            groups[key].push_back({sa, nwg});
-                            glds[key] = std::max(glds[key], lds);
+                            const std::array<int, 3> key{d->real ? 1 : 0, sh.nq, sh.nr};
+                            groups[key].push_back({sa, sh.nwg});
+                            const size_t lds = gshape.count(key) ? gshape[key].lds : 0;
+                            gshape[key] = sh;
+                            gshape[key].lds = std::max(sh.lds, lds);
                         } else {
                             stage_solve(*c, i, *d);
                         }
@@ -3332,8 +3434,10 @@ void ens_capture_lockstep(coral_amd_ensemble &e) {
                         tot += v[k].second;
                     }
                     e.lk_start_h[so + v.size()] = tot;
-                    if (!launch_solve16_batch(st, gp.first.first != 0, gp.first.second, tot, glds[gp.first],
-                                              e.lk_args.p + ao, e.lk_start.p + so, int(v.size())))
+                    Solve16Shape sh = gshape[gp.first];
+                    sh.nwg = tot;
+                    if (!launch_solve16_batch(st, gp.first[0] != 0, sh, e.lk_args.p + ao, e.lk_start.p + so,
+                                              int(v.size())))
                         throw std::runtime_error("batched 16-lane solve rejected its launches");
                     ao += v.size();
                     so += v.size() + 1;

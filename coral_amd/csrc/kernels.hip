@@ -1390,7 +1390,8 @@ __global__ __launch_bounds__(64) void k_factor(FactorArgs a) {
     // a whole system
     const bool l16 = a.ncol16 > 0;
     const int nb = l16 ? a.nblk : 1;
-    const int Sl = blockIdx.x, S = a.s0 + Sl, s = S / nb, blk = S - s * nb;
+    const int Sl = blockIdx.x, S = a.s0 + Sl, blk = S % nb;
+    const int s = a.rep ? a.rep[S / nb] : S / nb;
     const int N = a.total, w = a.nl + a.nu + 1;
     const int n = l16 ? a.blk_n : N, kl = l16 ? a.blk_nl : a.nl, ku = l16 ? a.blk_nu : a.nu;
     const int kv = kl + ku, ldab = 2 * kl + ku + 1;
@@ -1743,8 +1744,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // kernel held 137 VGPRs, now 86.)
 // Small grids are bound by the chain of steps of one wavefront: 64 x 64 x 33
 // 43 -> 31 us per launch, 72 x 48 x 41 54 -> 37, over both sweeps.  From
-// 128^2 x 65 on the launch moves its bytes at 4.0 to 4.4 TB/s, what a device
-// copy reaches, and did not change (256^2 x 129: 1.51 ms).
+// 128^2 x 65 on a launch with factors of its own for every system moves its
+// bytes at 4.0 to 4.4 TB/s, what a device copy reaches (256^2 x 129: 1.51 ms);
+// sharing factors between related systems takes 1.51 -> 0.87 ms there with two
+// systems each (the rotating recipe), 0.85 with four (the non-rotating one),
+// 0.44 -> 0.25 at 192^2 x 65, 0.21 -> 0.14 at 128^2 x 65, bound by the vector
+// instructions of the steps.
 // ---------------------------------------------------------------------------
 // row_newbcast writes every lane of the row, so no old value is needed
 template <int T_>
@@ -1772,11 +1777,14 @@ __device__ inline double bperm_d(int addr, double v) {
 }
 __device__ inline double2 bperm_c(int addr, double2 v) { return make_double2(bperm_d(addr, v.x), bperm_d(addr, v.y)); }
 
-// Position words of a block (see Solve16Args::words): row of the system at
-// bits 0-14, column at 15-29 (SOLVE16_NONE: padding), rotation of the
-// right-hand side (psi) at bit 30, of the solution (phi) at bit 31.
-__device__ inline int w_row(unsigned w) { return int(w & 0x7FFFu); }
-__device__ inline int w_col(unsigned w) { return int((w >> 15) & 0x7FFFu); }
+// Position words of a block (see solve16_words)
+__device__ inline int w_row(unsigned w) { return int(w & 0x3FFFu); }
+__device__ inline int w_col(unsigned w) { return int((w >> 14) & 0x3FFFu); }
+__device__ inline double2 flip(double2 v, unsigned neg) {
+    const unsigned m = neg << 31;
+    return make_double2(__hiloint2double(int(unsigned(__double2hiint(v.x)) ^ m), __double2loint(v.x)),
+                        __hiloint2double(int(unsigned(__double2hiint(v.y)) ^ m), __double2loint(v.y)));
+}
 
 // Loads: multipliers are read once and streamed (non-temporal); the U
 // windows of consecutive backward steps overlap in cache lines and use
@@ -1806,28 +1814,35 @@ __device__ inline T buf_load(const T *base, int nelem, unsigned byteoff) {
 // the compiler hoists the load, gives it a fresh register and copies it into
 // place at the end of the loop, and that copy waits for every load issued
 // since.
-template <typename T, int NQ, int PFB>
+template <typename T, int NQ, int PFB, int NR>
 struct Solve16 {
     // step j's U entries sit in ring slot (j mod 16) mod PFB and are reloaded
     // for step j - PFB, whose slot must be the same
     static_assert(PFB > 0 && 16 % PFB == 0, "the backward prefetch distance must divide 16");
     // forward step t of a block, then the prefetch of the next block's
-    // coefficient.  cur: the lane's window slot, inc: the rows that enter at
-    // this block's steps, yo collects y.  SEL: kl = 16 (see split_factors16).
-    // lo is the lane's position in its row, opaque to the compiler so that the
-    // lane masks are formed where they are used.
+    // coefficient.  For each of the NR right-hand sides cur is the lane's window
+    // slot, inc the rows that enter at this block's steps, and yo collects y.
+    // SEL: kl = 16 (see split_factors16).  lo is the lane's position in its row,
+    // opaque to the compiler so that the lane masks are formed where they are
+    // used.
     template <bool SEL, int t>
-    __device__ static inline void fwd_step(double2 &cur, double2 inc, double2 &yo, const uint4 &pv, T (&ring)[16],
-                                           const T *Lg, unsigned &lrec, int lo, int rowbase, int klp) {
+    __device__ static inline void fwd_step(double2 (&cur)[NR], const double2 (&inc)[NR], double2 (&yo)[NR],
+                                           const uint4 &pv, T (&ring)[16], const T *Lg, unsigned &lrec, int lo,
+                                           int rowbase, int klp) {
         const unsigned pw = t < 4 ? pv.x : t < 8 ? pv.y : t < 12 ? pv.z : pv.w;
         const int sig = int((pw >> (8 * (t & 3))) & 0xffu);
-        const double2 a = bcast16_c<t>(inc);
-        double2 yj = bperm_c((rowbase + (SEL ? sig & 15 : sig)) << 2, cur);
-        if (SEL) yj = csel(sig == 16, a, yj);   // the entering row is the pivot
-        cur = csel(lo == sig, a, cur);
-        cur = submul(cur, ring[t], yj);
-        yo = csel(lo == t, yj, yo);
-        asm volatile("" : "+v"(lrec) : "v"(cur.x), "v"(cur.y));
+        const int from = (rowbase + (SEL ? sig & 15 : sig)) << 2;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const double2 a = bcast16_c<t>(inc[k]);
+            double2 yj = bperm_c(from, cur[k]);
+            if (SEL) yj = csel(sig == 16, a, yj);   // the entering row is the pivot
+            cur[k] = csel(lo == sig, a, cur[k]);
+            cur[k] = submul(cur[k], ring[t], yj);
+            yo[k] = csel(lo == t, yj, yo[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < NR; ++k) asm volatile("" : "+v"(lrec) : "v"(cur[k].x), "v"(cur[k].y));
         ring[t] = ld_nt(Lg + (size_t)lrec + t * 4 * klp);
         __builtin_amdgcn_sched_barrier(0);   // and not later: the prefetch distance stays 16 steps
     }
@@ -1835,8 +1850,9 @@ struct Solve16 {
     // Lg: the wavefront's multiplier records (uniform); lrec: the offset of
     // the lane's entry of the next block's first column
     template <bool SEL, int t>
-    __device__ static inline void fwd_block(double2 &cur, double2 inc, double2 &yo, const uint4 &pv, T (&ring)[16],
-                                            const T *Lg, unsigned &lrec, int lo, int rowbase, int klp) {
+    __device__ static inline void fwd_block(double2 (&cur)[NR], const double2 (&inc)[NR], double2 (&yo)[NR],
+                                            const uint4 &pv, T (&ring)[16], const T *Lg, unsigned &lrec, int lo,
+                                            int rowbase, int klp) {
         fwd_step<SEL, t>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
         if constexpr (t < 15) fwd_block<SEL, t + 1>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
     }
@@ -1853,18 +1869,25 @@ struct Solve16 {
     // matrix and position, (m - 4 lo) entries.  Entry e = t - lo + 16q of
     // column j is U(j-1-k, j), k = e - 1, at cn.x + 4 e + m.
     template <int t>
-    __device__ static inline void bwd_step(double2 (&r)[NQ], double2 &xo, T (&cring)[PFB][NQ], const T *Ug, int2 cn,
-                                           unsigned &vm, int lo) {
+    __device__ static inline void bwd_step(double2 (&r)[NR][NQ], double2 (&xo)[NR], T (&cring)[PFB][NQ], const T *Ug,
+                                           int2 cn, unsigned &vm, int lo) {
         constexpr int slot = t % PFB;
-        const double2 xj = scale(bcast16_c<t>(r[0]), bcast16<t>(cring[slot][0]));
-        xo = csel(lo == t, xj, xo);
+        const T dinv = bcast16<t>(cring[slot][0]);
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) r[q] = submul(r[q], cring[slot][q], xj);
+        for (int k = 0; k < NR; ++k) {
+            const double2 xj = scale(bcast16_c<t>(r[k][0]), dinv);
+            xo[k] = csel(lo == t, xj, xo[k]);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) r[k][q] = submul(r[k][q], cring[slot][q], xj);
+        }
         // prefetch column j - PFB (its position in its block: (t - PFB) mod 16)
         constexpr int tn = (t - PFB) & 15;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(vm) : "v"(r[q].x), "v"(r[q].y));
-        asm volatile("" : "+v"(vm) : "v"(xo.x), "v"(xo.y));
+        for (int k = 0; k < NR; ++k) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(vm) : "v"(r[k][q].x), "v"(r[k][q].y));
+            asm volatile("" : "+v"(vm) : "v"(xo[k].x), "v"(xo[k].y));
+        }
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
             cring[slot][q] = buf_load(Ug + cn.x, 4 * cn.y, vm + unsigned((tn + 16 * q) * 4 * sizeof(T)));
@@ -1872,69 +1895,94 @@ struct Solve16 {
     }
 
     template <int t>
-    __device__ static inline void bwd_block(double2 (&r)[NQ], double2 &xo, T (&cring)[PFB][NQ], const T *Ug,
+    __device__ static inline void bwd_block(double2 (&r)[NR][NQ], double2 (&xo)[NR], T (&cring)[PFB][NQ], const T *Ug,
                                             const int2 (&cl)[16], unsigned &vm, int lo) {
         bwd_step<t>(r, xo, cring, Ug, cl[t], vm, lo);
         if constexpr (t > 0) bwd_block<t - 1>(r, xo, cring, Ug, cl, vm, lo);
     }
 };
 
-// the solve of one 64-lane workgroup wg of a launch (four block matrices)
-template <typename T, int NQ, int PFB>
+// the solve of workgroup (one wavefront) wg of a launch: four block matrices (a
+// group of records) and NR of the right-hand sides that share their factors.
+// The nslot / NR workgroups of a group follow each other eight apart, so that
+// they run on one XCD at about the same time and share its L2.  (As wavefronts
+// of one workgroup they shared SIMDs where others idled: 72 x 48 x 41 took 48 us
+// per launch instead of 38.)
+template <typename T, int NQ, int PFB, int NR>
 __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
-    using S = Solve16<T, NQ, PFB>;
-    extern __shared__ unsigned sW[];   // position words of every block
+    using S = Solve16<T, NQ, PFB, NR>;
+    extern __shared__ unsigned sW[];   // position words of the wavefront's slots, every block
     const T *__restrict__ L16 = reinterpret_cast<const T *>(a.L16);
     const T *__restrict__ Ur = reinterpret_cast<const T *>(a.U);
     const int n = a.n, ncol16 = a.ncol16;
     const int lane = threadIdx.x, l = lane & 15, rowbase = lane & 48;
-    const int wstride = n + 2 * SOLVE16_WPAD;
-    for (int e = lane; e < a.nblk * wstride; e += 64) sW[e] = a.words[e];
+    const int per = a.nslot / NR, chunk = wg / (8 * per), in = wg - chunk * (8 * per);
+    const int g = chunk * 8 + (in & 7), slot0 = NR * (in >> 3);   // group, first slot
     // factored matrix (structural block) of this 16-lane row
     const int nmat = a.nsys * a.nblk;
-    const int sg = wg * 4 + (lane >> 4);
-    const bool live = sg < nmat;
-    const int M = live ? sg : nmat - 1;
-    const int sys = M / a.nblk, blk = M - sys * a.nblk;
-    // the kxky (0,0) system is factored as the identity in block coordinates,
-    // which maps block position i to row w_row and column w_col; it solves
-    // x = rhs when its right-hand side is read at the columns too
-    const bool idsys = a.ident0 && sys == 0;
-    const bool dorot = a.rotate && !idsys;
-    // the wavefront's four matrices are one group of records (uniform)
-    const int g = wg, m = M & 3;
+    const int sg = g * 4 + (lane >> 4);
+    if (g * 4 >= nmat) return;
+    const int wstride = n + 2 * SOLVE16_WPAD, wslot = a.nblk * wstride;
+    for (int e = lane; e < NR * wslot; e += 64) sW[e] = a.words[slot0 * wslot + e];
+    const int M = sg < nmat ? sg : nmat - 1;
+    const int fsys = M / a.nblk, blk = M - fsys * a.nblk;
+    const int m = M & 3;
     const int klp = solve16_klp(a.kl);
     const T *Lg = L16 + (size_t)g * ncol16 * 4 * klp;   // wavefront's records; matrix m's column j at (4j + m)*klp
     const int B = (n + 15) >> 4;
-    // pivot offsets of block b: 16 bytes at P[b] (zero past n)
+    // pivot slots of block b: 16 bytes at P[b] (zero past n)
     const uint4 *P = reinterpret_cast<const uint4 *>(a.piv + (size_t)M * B * 16);
-    const double2 *b = a.rhs + (size_t)sys * a.total;
-    double2 *y = a.x + (size_t)sys * a.total;
     double2 *sink = a.sink + lane;   // stores of padding positions and idle lanes
+    // per right-hand side: its system (a slot without one repeats the first
+    // and writes nothing), operands and words
+    bool live[NR], idsys[NR], dorot[NR];
+    const double2 *b[NR];
+    double2 *y[NR];
+    const unsigned *W[NR];   // W[k][i]: position i (padding outside [0, n))
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+        int sys = a.mem ? a.mem[(size_t)fsys * a.nslot + slot0 + k] : fsys;
+        live[k] = sg < nmat && sys >= 0;
+        if (sys < 0) sys = a.mem[(size_t)fsys * a.nslot];
+        // the kxky (0,0) system is factored as the identity in block
+        // coordinates, which maps block position i to row w_row and column
+        // w_col; it solves x = rhs when its right-hand side is read at the
+        // columns too
+        idsys[k] = a.ident0 && sys == 0;
+        dorot[k] = a.rotate && !idsys[k];
+        b[k] = a.rhs + (size_t)sys * a.total;
+        y[k] = a.x + (size_t)sys * a.total;
+        W[k] = sW + (k * a.nblk + blk) * wstride + SOLVE16_WPAD;
+    }
     __syncthreads();
-    const unsigned *W = sW + blk * wstride + SOLVE16_WPAD;   // W[i]: position i (padding outside [0, n))
-    auto code = [&](unsigned w) -> int { return dorot ? int(w >> 30) : 0; };
-    auto src_row = [&](unsigned w) -> int { return idsys ? w_col(w) : w_row(w); };
-    auto row_or0 = [&](unsigned w) -> int { const int r = src_row(w); return r != SOLVE16_NONE ? r : 0; };
+    auto code = [&](int k, unsigned w) -> int { return dorot[k] ? int(w >> 30) : 0; };
+    auto src_row = [&](int k, unsigned w) -> int { return idsys[k] ? w_col(w) : w_row(w); };
+    auto row_or0 = [&](int k, unsigned w) -> int { const int r = src_row(k, w); return r != SOLVE16_NONE ? r : 0; };
     auto col_or0 = [&](unsigned w) -> int { const int c = w_col(w); return c != SOLVE16_NONE ? c : 0; };
-    auto fix_rhs = [&](double2 v, unsigned w) -> double2 {
-        return rot_in(csel(src_row(w) != SOLVE16_NONE, v, make_double2(0.0, 0.0)), code(w));
+    auto fix_rhs = [&](int k, double2 v, unsigned w) -> double2 {
+        const double2 s = flip(v, idsys[k] ? 0u : (w >> 28) & 1u);
+        return rot_in(csel(src_row(k, w) != SOLVE16_NONE, s, make_double2(0.0, 0.0)), code(k, w));
     };
     auto fix_y = [&](double2 v, unsigned w) -> double2 {
         return csel(w_col(w) != SOLVE16_NONE, v, make_double2(0.0, 0.0));
     };
-    auto out_ptr = [&](unsigned w) -> double2 * {
+    auto out_ptr = [&](int k, unsigned w) -> double2 * {
         const int c = w_col(w);
-        return (live && c != SOLVE16_NONE) ? y + c : sink;
+        return (live[k] && c != SOLVE16_NONE) ? y[k] + c : sink;
     };
 
     // ---- forward ----
     auto forward = [&](auto sel) {
         constexpr bool SEL = decltype(sel)::value;
         const int D = solve16_window(a.kl);   // rows in the window; row D + 16 b + l enters at step l of block b
-        const unsigned w0 = W[l], w1 = W[D + l];
-        double2 cur = csel(l < D, fix_rhs(b[row_or0(w0)], w0), make_double2(0.0, 0.0)), yo = make_double2(0.0, 0.0);
-        double2 inc = fix_rhs(b[row_or0(w1)], w1);
+        double2 cur[NR], yo[NR], inc[NR];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const unsigned w0 = W[k][l], w1 = W[k][D + l];
+            cur[k] = csel(l < D, fix_rhs(k, b[k][row_or0(k, w0)], w0), make_double2(0.0, 0.0));
+            inc[k] = fix_rhs(k, b[k][row_or0(k, w1)], w1);
+            yo[k] = make_double2(0.0, 0.0);
+        }
         uint4 pv = P[0];
         T ring[16];
         // the lane's entry of a record (lanes past the window read the last one)
@@ -1949,13 +1997,21 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
             asm volatile("" : "+v"(lo));
             // loaded here, consumed at the end of this block: the rows that
             // enter in block bk+1 and its pivots
-            const unsigned w2 = W[bk * 16 + 16 + D + l];
-            const double2 nx2 = b[row_or0(w2)];
+            unsigned w2[NR];
+            double2 nx2[NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                w2[k] = W[k][bk * 16 + 16 + D + l];
+                nx2[k] = b[k][row_or0(k, w2[k])];
+            }
             const uint4 pvn = P[min(bk + 1, B - 1)];
             unsigned lrec = lbase + unsigned(bk * 16 + 16) * unsigned(4 * klp);
             S::template fwd_block<SEL, 0>(cur, inc, yo, pv, ring, Lg, lrec, lo, rowbase, klp);
-            *out_ptr(W[bk * 16 + l]) = yo;   // intermediate, kept at the unknown's slot
-            inc = fix_rhs(nx2, w2);
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                *out_ptr(k, W[k][bk * 16 + l]) = yo[k];   // intermediate, kept at the unknown's slot
+                inc[k] = fix_rhs(k, nx2[k], w2[k]);
+            }
             pv = pvn;
         }
     };
@@ -1978,11 +2034,15 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
         const unsigned long long w = ucol[k];
         return make_int2(int(unsigned(w)), int(unsigned(w >> 32)));
     };
-    double2 r[NQ];
+    double2 r[NR][NQ], xo[NR];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const unsigned wq = W[(B - 1 - q) * 16 + l];
-        r[q] = fix_y(y[col_or0(wq)], wq);
+    for (int k = 0; k < NR; ++k) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const unsigned wq = W[k][(B - 1 - q) * 16 + l];
+            r[k][q] = fix_y(y[k][col_or0(wq)], wq);
+        }
+        xo[k] = make_double2(0.0, 0.0);
     }
     T cring[PFB][NQ];
     const unsigned vm0 = unsigned((m - 4 * l) * int(sizeof(T)));
@@ -1997,65 +2057,99 @@ __device__ __forceinline__ void solve16_body(const Solve16Args &a, int wg) {
         // same way whether it is entered from here or from its own end
         __builtin_amdgcn_sched_barrier(0);
     }
-    double2 xo = make_double2(0.0, 0.0);
     for (int bk = B - 1; bk >= 0; --bk) {
         int lo = l;
         asm volatile("" : "+v"(lo));
         // loaded here, consumed at the end of this block: the forward result of
         // block bk-NQ, which enters the window of blocks being updated
-        const unsigned wy = W[(bk - NQ) * 16 + l];
-        const double2 ynx = y[col_or0(wy)];
+        unsigned wy[NR];
+        double2 ynx[NR];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            wy[k] = W[k][(bk - NQ) * 16 + l];
+            ynx[k] = y[k][col_or0(wy[k])];
+        }
         // columns 16 bk - PFB .. 16 bk + 15 - PFB, fetched during this block
         int2 cl[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) cl[t] = column(bk * 16 + t);
         unsigned vm = vm0;
         S::template bwd_block<15>(r, xo, cring, Ug, cl, vm, lo);
-        const unsigned w0 = W[bk * 16 + l];
-        *out_ptr(w0) = rot_out(xo, code(w0));
 #pragma unroll
-        for (int q = 0; q < NQ - 1; ++q) r[q] = r[q + 1];
-        r[NQ - 1] = fix_y(ynx, wy);
+        for (int k = 0; k < NR; ++k) {
+            const unsigned w0 = W[k][bk * 16 + l];
+            *out_ptr(k, w0) = flip(rot_out(xo[k], code(k, w0)), idsys[k] ? 0u : (w0 >> 29) & 1u);
+#pragma unroll
+            for (int q = 0; q < NQ - 1; ++q) r[k][q] = r[k][q + 1];
+            r[k][NQ - 1] = fix_y(ynx[k], wy[k]);
+        }
     }
 }
 
-template <typename T, int NQ, int PFB>
+template <typename T, int NQ, int PFB, int NR>
 __global__ __launch_bounds__(64) void k_solve16(Solve16Args a) {
-    solve16_body<T, NQ, PFB>(a, blockIdx.x);
+    solve16_body<T, NQ, PFB, NR>(a, blockIdx.x);
 }
 
 // Solves of several launches in one: workgroup b belongs to the launch r with
 // start[r] <= b < start[r + 1] (nrun launches, their arguments in args) and
 // runs as that launch's workgroup b - start[r]
-template <typename T, int NQ, int PFB>
+template <typename T, int NQ, int PFB, int NR>
 __global__ __launch_bounds__(64) void k_solve16_batch(const Solve16Args *__restrict__ args,
                                                       const int *__restrict__ start, int nrun) {
     const int b = blockIdx.x;
     int r = 0;
     while (r + 1 < nrun && start[r + 1] <= b) ++r;
     const Solve16Args a = args[r];
-    solve16_body<T, NQ, PFB>(a, b - start[r]);
+    solve16_body<T, NQ, PFB, NR>(a, b - start[r]);
+}
+
+bool solve16_shape(const Solve16Args &a, Solve16Shape &sh) {
+    if (a.kl > 16 || a.n < 32 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol || !a.sink) return false;
+    if (a.nslot < 1 || a.nslot > SOLVE16_SLOTS || (a.nslot > 1 && !a.mem)) return false;
+    sh.nq = 1 + (a.kv + 15) / 16;
+    if (sh.nq < 2 || sh.nq > 4) return false;
+    // Two right-hand sides per wavefront read the factors once for both and
+    // share the step's masks and addresses, but take 1.35 times one's chain of
+    // steps: below a wavefront per SIMD (1024) that chain is the launch time.
+    // One against two, us per launch with four sharing: 64 x 64 x 33 (504
+    // wavefronts of two) 31, 39; 96 x 96 x 48 (1140) 84, 72; 128 x 128 x 65 182,
+    // 139; 256 x 256 x 129 1235, 851.
+    const int groups = (a.nsys * a.nblk + 3) / 4;
+    sh.nr = a.nslot % 2 == 0 && groups * (a.nslot / 2) >= 1024 ? 2 : 1;
+    sh.nwg = (groups + 7) / 8 * 8 * (a.nslot / sh.nr);
+    sh.lds = size_t(sh.nr) * a.nblk * (a.n + 2 * SOLVE16_WPAD) * sizeof(unsigned);
+    return sh.lds <= 32768;
+}
+
+// calls f with the kernel template's NQ and NR as constants
+template <class F>
+static bool solve16_variant(const Solve16Shape &sh, F &&f) {
+    auto nq = [&](auto nr) {
+        switch (sh.nq) {
+        case 2: f(std::integral_constant<int, 2>{}, nr); return true;
+        case 3: f(std::integral_constant<int, 3>{}, nr); return true;
+        case 4: f(std::integral_constant<int, 4>{}, nr); return true;
+        default: return false;
+        }
+    };
+    return sh.nr == 2 ? nq(std::integral_constant<int, 2>{}) : nq(std::integral_constant<int, 1>{});
 }
 
 template <typename T>
 static bool launch_solve16(hipStream_t st, const Solve16Args &a) {
-    if (a.kl > 16 || a.n < 32 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol) return false;
-    const int nq = 1 + (a.kv + 15) / 16;
-    const dim3 grid((a.nsys * a.nblk + 3) / 4);
-    const size_t lds = size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) * sizeof(unsigned);
-    if (lds > 32768 || !a.sink) return false;
-    switch (nq) {
-    case 2: hipLaunchKernelGGL((k_solve16<T, 2, 8>), grid, dim3(64), lds, st, a); break;
-    case 3: hipLaunchKernelGGL((k_solve16<T, 3, 8>), grid, dim3(64), lds, st, a); break;
-    case 4: hipLaunchKernelGGL((k_solve16<T, 4, 8>), grid, dim3(64), lds, st, a); break;
-    default: return false;
-    }
+    Solve16Shape sh;
+    if (!solve16_shape(a, sh)) return false;
+    const bool ok = solve16_variant(sh, [&](auto nq, auto nr) {
+        hipLaunchKernelGGL((k_solve16<T, decltype(nq)::value, SOLVE16_UPAD, decltype(nr)::value>), dim3(sh.nwg),
+                           dim3(64), sh.lds, st, a);
+    });
     CHECK_LAUNCH();
-    return true;
+    return ok;
 }
 
 std::vector<unsigned> solve16_words(int total, int nblk, int blk_n, const int *blk_row, const int *blk_col,
-                                    const unsigned char *rot) {
+                                    const unsigned char *rot, const Solve16Sym *sym) {
     const size_t stride = size_t(blk_n) + 2 * SOLVE16_WPAD;
     std::vector<unsigned> w(size_t(nblk) * stride, SOLVE16_NOWORD);
     for (int b = 0; b < nblk; ++b)
@@ -2063,7 +2157,10 @@ std::vector<unsigned> solve16_words(int total, int nblk, int blk_n, const int *b
             const size_t e = size_t(b) * blk_n + i;
             const int r = blk_row ? blk_row[e] : (i < total ? i : -1);
             const int c = blk_col ? blk_col[e] : (i < total ? i : -1);
-            unsigned v = unsigned(r < 0 ? SOLVE16_NONE : r) | (unsigned(c < 0 ? SOLVE16_NONE : c) << 15);
+            unsigned v = unsigned(r < 0 ? SOLVE16_NONE : sym ? sym->row[r] : r) |
+                         (unsigned(c < 0 ? SOLVE16_NONE : sym ? sym->col[c] : c) << 14);
+            if (sym && r >= 0) v |= unsigned(sym->rneg[r] & 1) << 28;
+            if (sym && c >= 0) v |= unsigned(sym->cneg[c] & 1) << 29;
             if (rot && r >= 0) v |= unsigned(rot[r] & 1) << 30;
             if (rot && c >= 0) v |= unsigned((rot[c] >> 1) & 1) << 31;
             w[size_t(b) * stride + SOLVE16_WPAD + i] = v;
@@ -2141,39 +2238,24 @@ void solve16_trim_u_copy(hipStream_t st, const void *Ufull, int elem, int n, int
 }
 
 int solve16_ncol(int n, int kl, int kv) {
-    // (positions are packed in 15 bits of the position words)
+    // (positions are packed in 14 bits of the position words)
     if (kl > 16 || n < 32 || n >= SOLVE16_NONE || 1 + (kv + 15) / 16 > 4) return 0;
     return 16 * ((n + 15) / 16 + 1);
 }
 
-bool solve16_shape(const Solve16Args &a, int &nwg, size_t &lds, int &nq) {
-    if (a.kl > 16 || a.n < 32 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol || !a.sink) return false;
-    nq = 1 + (a.kv + 15) / 16;
-    if (nq < 2 || nq > 4) return false;
-    nwg = (a.nsys * a.nblk + 3) / 4;
-    lds = size_t(a.nblk) * (a.n + 2 * SOLVE16_WPAD) * sizeof(unsigned);
-    return lds <= 32768;
-}
-
-bool launch_solve16_batch(hipStream_t st, bool real, int nq, int nwg, size_t lds, const Solve16Args *args,
-                          const int *start, int nrun) {
-    if (nwg <= 0 || nrun <= 0 || lds > 32768) return false;
-    const dim3 grid{unsigned(nwg)};
-#define SOLVE16_BATCH(T_)                                                                                         \
-    switch (nq) {                                                                                                 \
-    case 2: hipLaunchKernelGGL((k_solve16_batch<T_, 2, 8>), grid, dim3(64), lds, st, args, start, nrun); break;  \
-    case 3: hipLaunchKernelGGL((k_solve16_batch<T_, 3, 8>), grid, dim3(64), lds, st, args, start, nrun); break;  \
-    case 4: hipLaunchKernelGGL((k_solve16_batch<T_, 4, 8>), grid, dim3(64), lds, st, args, start, nrun); break;  \
-    default: return false;                                                                                        \
-    }
-    if (real) {
-        SOLVE16_BATCH(double)
-    } else {
-        SOLVE16_BATCH(double2)
-    }
-#undef SOLVE16_BATCH
+bool launch_solve16_batch(hipStream_t st, bool real, const Solve16Shape &sh, const Solve16Args *args, const int *start,
+                          int nrun) {
+    if (sh.nwg <= 0 || nrun <= 0 || sh.lds > 32768) return false;
+    auto go = [&](auto one) {
+        using T = decltype(one);
+        return solve16_variant(sh, [&](auto nq, auto nr) {
+            hipLaunchKernelGGL((k_solve16_batch<T, decltype(nq)::value, SOLVE16_UPAD, decltype(nr)::value>),
+                               dim3(unsigned(sh.nwg)), dim3(64), sh.lds, st, args, start, nrun);
+        });
+    };
+    const bool ok = real ? go(double{}) : go(double2{});
     CHECK_LAUNCH();
-    return true;
+    return ok;
 }
 
 bool launch_solve16_real(hipStream_t st, const Solve16Args &a) { return launch_solve16<double>(st, a); }

@@ -269,6 +269,7 @@ struct FactorArgs {
     // (block index = s*nblk + b).  nblk = 1 with null maps: the whole system.
     int nblk, blk_n, blk_nl, blk_nu;
     const int *blk_row, *blk_col;
+    const int *rep;           // systems factored (null: all); s0/ns and the outputs count them
 };
 void launch_factor(hipStream_t st, const FactorArgs &a);
 // generic batched factorization of LAPACK band input (for the unit seam)
@@ -297,9 +298,13 @@ constexpr int SOLVE16_PAD = 2048;
 // columns before the first in the solve's table of trimmed U records: the
 // backward sweep fetches that many steps ahead
 constexpr int SOLVE16_UPAD = 8;
-// 16-lane solve of nsys systems of `total` unknowns, each made of nblk
-// structural blocks of n unknowns and band (kl, kv - kl) (see FactorArgs);
-// factors in the layout k_factor writes for ncol16 > 0.
+// 16-lane solve with nsys factored systems of `total` unknowns, each made of
+// nblk structural blocks of n unknowns and band (kl, kv - kl) (see FactorArgs);
+// factors in the layout k_factor writes for ncol16 > 0.  Systems related by a
+// symmetry (SystemTables::Symmetry) share their factors: factored system i
+// serves the up to nslot systems mem[i*nslot + k] (-1: none), the k-th through
+// word table k.
+constexpr int SOLVE16_SLOTS = 4;
 struct Solve16Args {
     const void *L16;             // double (real form) or double2
     // U records trimmed per column (solve16_trim_u_copy): for wavefront group
@@ -310,9 +315,11 @@ struct Solve16Args {
     long long ustride;
     int ncol16;
     const unsigned char *piv;    // [nsys*nblk][16*ceil(n/16)] window slots of the pivots, zero past n
-    // position words (solve16_words): row and column of the system at each
-    // position of a block, and their real-form rotations
+    // position words (solve16_words), one table per slot: row and column of the
+    // system at each position of a block, their signs and real-form rotations
     const unsigned *words;
+    const int *mem;              // null: factored system i serves system i
+    int nslot;
     int rotate;                  // apply the rotations (real form)
     int ident0;                  // system 0 is the identity and is not rotated
     int total, n, kl, kv, nsys, nblk;
@@ -334,26 +341,37 @@ void solve16_trim_u_copy(hipStream_t st, const void *Ufull, int elem, int n, int
                          long long ustride, void *Utrim);
 // "no row / column" in a position word (padding of a block), and the word of
 // a position outside the block
-constexpr int SOLVE16_NONE = 0x7FFF;
-constexpr unsigned SOLVE16_NOWORD = 0x3FFFFFFFu;
-// words of padding on each side of a block's words (the solve reads up to 96
-// positions before and 79 after the block)
-constexpr int SOLVE16_WPAD = 128;
+constexpr int SOLVE16_NONE = 0x3FFF;
+constexpr unsigned SOLVE16_NOWORD = 0x0FFFFFFFu;
+// words of padding on each side of a block's words (the solve reads up to 64
+// positions before and 47 after the block)
+constexpr int SOLVE16_WPAD = 64;
 // Position words of the nblk blocks of blk_n positions (blk_row/blk_col as in
 // FactorArgs, null for one block of the whole system; rot as in SystemTables,
-// or null): row | col << 15 | psi(row) << 30 | phi(col) << 31, block b at
+// or null; sym: the member's symmetry, or null): row | col << 14 | negative
+// row << 28 | negative column << 29 | psi(row) << 30 | phi(col) << 31, block b at
 // b*(blk_n + 2*SOLVE16_WPAD) + SOLVE16_WPAD, padding SOLVE16_NOWORD.
+struct Solve16Sym {
+    std::vector<int> row, col;
+    std::vector<unsigned char> rneg, cneg;
+};
 std::vector<unsigned> solve16_words(int total, int nblk, int blk_n, const int *blk_row, const int *blk_col,
-                                    const unsigned char *rot);
-// workgroups, LDS bytes and NQ of the 16-lane solve of a (false: it does not take a)
-bool solve16_shape(const Solve16Args &a, int &nwg, size_t &lds, int &nq);
+                                    const unsigned char *rot, const Solve16Sym *sym = nullptr);
+// launch shape of the 16-lane solve of a: workgroups (of 64), LDS bytes,
+// registers per window (nq) and right-hand sides per wavefront (nr)
+struct Solve16Shape {
+    int nwg, nq, nr;
+    size_t lds;
+};
+// (false: the solve does not take a)
+bool solve16_shape(const Solve16Args &a, Solve16Shape &sh);
 // the 16-lane solves of nrun launches of one element type (real: the real
-// form; complex entries must carry rotate = 0) and NQ in one launch: device
-// copies of their arguments and of start[0..nrun] (cumulative workgroups),
-// nwg = start[nrun] workgroups, lds the largest of theirs; results equal each
-// launch's own
-bool launch_solve16_batch(hipStream_t st, bool real, int nq, int nwg, size_t lds, const Solve16Args *args,
-                          const int *start, int nrun);
+// form; complex entries must carry rotate = 0) and one shape (nq, nr) in one
+// launch: device copies of their arguments and of start[0..nrun]
+// (cumulative workgroups), sh.nwg = start[nrun] workgroups, sh.lds the largest
+// of theirs; results equal each launch's own
+bool launch_solve16_batch(hipStream_t st, bool real, const Solve16Shape &sh, const Solve16Args *args, const int *start,
+                          int nrun);
 bool launch_solve16_real(hipStream_t st, const Solve16Args &a);
 bool launch_solve16_complex(hipStream_t st, const Solve16Args &a);
 // (ident0: system 0 is the identity and is not rotated)

@@ -262,6 +262,14 @@ class Solver:
               "coral_amd_factor_blocks")
         return tuple(x.value for x in v)
 
+    def factored_systems(self, isys: int = 0):
+        """(wavenumbers factored, most that share one factorization) of kxky
+        system `isys`."""
+        v = [ctypes.c_int32() for _ in range(2)]
+        check(lib.coral_amd_factored_systems(self._ctx, isys, *[ctypes.byref(x) for x in v]),
+              "coral_amd_factored_systems")
+        return tuple(x.value for x in v)
+
     def u_entries_per_column(self, isys: int = 0, kind: int = 0) -> float:
         """Mean number of U entries per column the solve reads (records cut to
         their longest nonzero prefix over all wavenumbers; after factorization)."""

@@ -163,6 +163,15 @@ int coral_amd_factor_kind(coral_amd_ctx *ctx, int32_t isys, int32_t *is_real);
 int coral_amd_factor_blocks(coral_amd_ctx *ctx, int32_t kind, int32_t isys, int32_t *nblk, int32_t *blk_n,
                             int32_t *blk_nl, int32_t *blk_nu, double *u_entries);
 
+/* Factored systems of kxky system isys.  The operators of many recipes are
+ * related between wavenumbers, (kx, ky) to (kx, -ky) by the reflection y -> -y
+ * and to (ky, -kx) by a quarter turn (equal box lengths), up to the order and
+ * signs of rows and columns; one factorization then serves up to nshare (1, 2
+ * or 4) wavenumbers, and nfactored of all kept ones are factored.
+ * CORAL_AMD_NO_SHARED_FACTORS=1 before coral_amd_create factors every one, as
+ * the reference does (PL_IMEX_timestepping.f90:351-422). */
+int coral_amd_factored_systems(coral_amd_ctx *ctx, int32_t isys, int32_t *nfactored, int32_t *nshare);
+
 /* Physical values of coupled variable ivar of system isys in the current state:
  * the volumes Coral writes to CheckPoints/QuickSave.{kxky,zero}.sysNNN.varNNN.rollingR
  * (export_checkpoints, PL_IMEX_timestepping_output.f90:388-455).  kind 0: C
