@@ -13,6 +13,8 @@
 #include <string>
 #include <vector>
 
+#include "hostcopy.hpp"
+
 #include "../../include/coral_amd.h"
 #include "assembly.hpp"
 #include "kernels.hpp"
@@ -55,6 +57,14 @@ struct DevBuf {
         alloc(v.size());
         if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     }
+};
+
+// device tables of one coupled variable: extraction rows (Chebyshev coefficients
+// of its Galerkin coefficients), and the square stencil's inverse with positions
+struct VarDev {
+    int ncol = 0;
+    DevBuf<int> rowptr, col, pos;
+    DevBuf<double> val, Sinv;
 };
 
 struct SysDev {
@@ -127,6 +137,12 @@ struct TimerRec {
 }  // namespace
 
 struct coral_amd_ctx {
+    // host copies: pinned chunks, and a device array in the host's layout
+    HostCopy host;
+    DevBuf<double2> hostd;
+    // stencil tables of coupled variables (coral_amd_get/set_variable_physical),
+    // built at a variable's first use
+    std::map<std::pair<int, int>, std::unique_ptr<VarDev>> var_dev;
     Problem P;
     int device = 0;
     hipStream_t stream = nullptr;
@@ -1735,16 +1751,93 @@ void ensure_phys(coral_amd_ctx &c) {
     if (c.physd.n != n) c.physd.alloc(n);
 }
 
+// out[b][c][r] = in[b][r][c] for r < R, c < C, through LDS tiles; ir, ib, oc, ob:
+// the strides of r and b in in, of c and b in out
+template <class TI, class TO>
+__global__ __launch_bounds__(256) void k_transpose(const TI *__restrict__ in, int R, int C, size_t ir, size_t ib,
+                                                   TO *__restrict__ out, size_t oc, size_t ob) {
+    __shared__ TI tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const unsigned nct = unsigned(C + 31) / 32, rt = blockIdx.x / nct;
+    const int c0 = int(blockIdx.x - rt * nct) * 32, r0 = int(rt) * 32;
+    in += blockIdx.y * ib;
+    out += blockIdx.y * ob;
+    for (int i = ty; i < 32; i += 8)
+        if (r0 + i < R && c0 + tx < C) tile[i][tx] = in[(r0 + i) * ir + c0 + tx];
+    __syncthreads();
+    for (int i = ty; i < 32; i += 8)
+        if (c0 + i < C && r0 + tx < R) {
+            if constexpr (std::is_same<TI, TO>::value)
+                out[(c0 + i) * oc + r0 + tx] = tile[tx][i];
+            else
+                out[(c0 + i) * oc + r0 + tx] = make_double2(tile[tx][i].x, tile[tx][i].y);
+        }
+}
+template <class TI, class TO>
+void transpose(hipStream_t st, const TI *in, int R, int C, size_t ir, size_t ib, TO *out, size_t oc, size_t ob, int nb) {
+    const long long tiles = (long long)((C + 31) / 32) * ((R + 31) / 32);
+    if (tiles > 2147483647LL || nb > 65535) throw std::runtime_error("transpose: grid too large");
+    hipLaunchKernelGGL((k_transpose<TI, TO>), dim3(unsigned(tiles), unsigned(nb)), dim3(256), 0, st, in, R, C, ir, ib,
+                       out, oc, ob);
+    check_launch("transpose");
+}
+
+// Host layouts are formed on the device and copied as they are: a volume's
+// transposition on one host core took longer than everything else about it.
+void ensure_hostd(coral_amd_ctx &c, size_t n) {
+    if (c.hostd.n < n) c.hostd.alloc(n);
+}
+
 // device [z][y][x] -> host [x][y][z]
 void download_phys(coral_amd_ctx &c, double *out) {
     const Problem &P = c.P;
-    HIP_OK(hipStreamSynchronize(c.stream));
-    std::vector<double> h(c.physd.n);
-    HIP_OK(hipMemcpy(h.data(), c.physd.p, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int z = 0; z < P.NZAA; ++z)
-        for (int y = 0; y < P.NYAA; ++y)
-            for (int x = 0; x < P.NXAA; ++x)
-                out[(size_t(x) * P.NYAA + y) * P.NZAA + z] = h[(size_t(z) * P.NYAA + y) * P.NXAA + x];
+    ensure_hostd(c, (c.physd.n + 1) / 2);
+    double *d = reinterpret_cast<double *>(c.hostd.p);
+    const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
+    transpose(c.stream, c.physd.p, P.NZAA, P.NXAA, NY * NX, NX, d, NY * NZ, NZ, P.NYAA);
+    c.host.to_host(c.stream, c.device, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return out + x * NY * NZ; },
+                   [](int, int) {});
+}
+
+// host [x][y][z] -> device [z][y][x]
+void upload_phys(coral_amd_ctx &c, const double *in) {
+    const Problem &P = c.P;
+    ensure_phys(c);
+    ensure_hostd(c, (c.physd.n + 1) / 2);
+    double *d = reinterpret_cast<double *>(c.hostd.p);
+    const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
+    c.host.to_device(c.stream, c.device, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return in + x * NY * NZ; });
+    transpose(c.stream, d, P.NXAA, P.NZAA, NY * NZ, NZ, c.physd.p, NY * NX, NX, P.NYAA);
+}
+
+// nf fields of nv values per kept wavenumber, device [field][s][value], to the
+// host's [field][ix][ky slot][value], dealiased slots zero
+void download_modes(coral_amd_ctx &c, const double2 *dev, int nf, int nv, double *out) {
+    const Problem &P = c.P;
+    const size_t nsys = P.nsys, row = size_t(nv) * sizeof(double2), line = size_t(P.NYAA) * row;
+    char *o = reinterpret_cast<char *>(out);
+    c.host.to_host(
+        c.stream, c.device, dev, nf * nsys, row,
+        [&](size_t r) {
+            const size_t f = r / nsys, s = r - f * nsys, ix = s / P.nky, jy = s - ix * P.nky;
+            return o + (f * P.nkx + ix) * line + P.ky_slot[jy] * row;
+        },
+        [&](int part, int parts) {
+            // the dealiased slots of a line follow the non-negative ky
+            for (size_t l = part; l < size_t(nf) * P.nkx; l += parts)
+                std::memset(o + l * line + (P.NY / 2) * row, 0, (P.NYAA - P.nky) * row);
+        });
+}
+
+// the kept wavenumbers of one field in the host's layout, to device [s][value]
+void upload_modes(coral_amd_ctx &c, const double *in, int nv, double2 *dev) {
+    const Problem &P = c.P;
+    const size_t row = size_t(nv) * sizeof(double2), line = size_t(P.NYAA) * row;
+    const char *h = reinterpret_cast<const char *>(in);
+    c.host.to_device(c.stream, c.device, dev, P.nsys, row, [&](size_t s) {
+        const size_t ix = s / P.nky, jy = s - ix * P.nky;
+        return h + ix * line + P.ky_slot[jy] * row;
+    });
 }
 
 int fail(const std::exception &e) {
@@ -1929,21 +2022,13 @@ int coral_amd_upload_state(coral_amd_ctx *c, int32_t kind, int32_t isys, const d
         // for the context's non-blocking streams: finish queued steps first
         HIP_OK(hipStreamSynchronize(c->stream));
         HIP_OK(hipStreamSynchronize(c->side));
-        const Problem &P = c->P;
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
             const int total = d.t->total;
-            std::vector<double2> h(size_t(P.nsys) * total);
-            for (int ix = 0; ix < P.nkx; ++ix)
-                for (int jy = 0; jy < P.nky; ++jy) {
-                    const int s = ix * P.nky + jy;
-                    const size_t src = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * total;
-                    for (int i = 0; i < total; ++i)
-                        h[size_t(s) * total + i] =
-                            (s == 0) ? make_double2(0.0, 0.0) : make_double2(data[2 * (src + i)], data[2 * (src + i) + 1]);
-                }
-            HIP_OK(hipMemcpy(d.field.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
+            upload_modes(*c, data, total, d.field.p);
+            fill_zero(c->stream, d.field.p, total);   // the (0, 0) mode
+            HIP_OK(hipStreamSynchronize(c->stream));
         } else if (kind == 1) {
             if (isys < 0 || isys >= int(c->zs.size())) throw std::runtime_error("bad mean system index");
             SysDev &d = *c->zs[isys];
@@ -1964,23 +2049,11 @@ int coral_amd_download_state(coral_amd_ctx *c, int32_t kind, int32_t isys, doubl
         if (!c || !data) throw std::runtime_error("null argument");
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        const Problem &P = c->P;
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
             const int total = d.t->total;
-            std::vector<double2> h(size_t(P.nsys) * total);
-            HIP_OK(hipMemcpy(h.data(), d.field.p, h.size() * sizeof(double2), hipMemcpyDeviceToHost));
-            std::memset(data, 0, sizeof(double) * 2 * size_t(P.nkx) * P.NYAA * total);
-            for (int ix = 0; ix < P.nkx; ++ix)
-                for (int jy = 0; jy < P.nky; ++jy) {
-                    const int s = ix * P.nky + jy;
-                    const size_t dst = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * total;
-                    for (int i = 0; i < total; ++i) {
-                        data[2 * (dst + i)] = h[size_t(s) * total + i].x;
-                        data[2 * (dst + i) + 1] = h[size_t(s) * total + i].y;
-                    }
-                }
+            download_modes(*c, d.field.p, 1, total, data);
         } else if (kind == 1) {
             if (isys < 0 || isys >= int(c->zs.size())) throw std::runtime_error("bad mean system index");
             SysDev &d = *c->zs[isys];
@@ -2217,6 +2290,33 @@ VarMaps var_maps(const SystemTables &t, int NZ, int v) {
     m.Sinv = B;
     return m;
 }
+
+// the variable's tables on the device, built at its first use
+const VarDev &var_dev(coral_amd_ctx &c, int isys, int ivar) {
+    auto &slot = c.var_dev[{isys, ivar}];
+    if (!slot) {
+        const VarMaps m = var_maps(*c.ks[isys]->t, c.P.NZ, ivar);
+        std::vector<int> rowptr(1, 0), col;
+        std::vector<double> val;
+        for (int n = 0; n < c.P.NZ; ++n) {
+            for (int j = 0; j < m.ncol; ++j)
+                if (m.S(n, j) != 0.0) {
+                    col.push_back(m.pos[j]);
+                    val.push_back(m.S(n, j));
+                }
+            rowptr.push_back(int(col.size()));
+        }
+        std::unique_ptr<VarDev> v(new VarDev());
+        v->ncol = m.ncol;
+        v->rowptr.upload(rowptr);
+        v->col.upload(col);
+        v->val.upload(val);
+        v->pos.upload(m.pos);
+        v->Sinv.upload(m.Sinv);
+        slot = std::move(v);
+    }
+    return *slot;
+}
 }  // namespace
 
 int coral_amd_get_variable_physical(coral_amd_ctx *c, int32_t kind, int32_t isys, int32_t ivar, double *out) {
@@ -2227,23 +2327,8 @@ int coral_amd_get_variable_physical(coral_amd_ctx *c, int32_t kind, int32_t isys
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
-            const VarMaps m = var_maps(*d.t, P.NZ, ivar);
-            std::vector<int> rowptr(1, 0), col;
-            std::vector<double> val;
-            for (int n = 0; n < P.NZ; ++n) {
-                for (int j = 0; j < m.ncol; ++j)
-                    if (m.S(n, j) != 0.0) {
-                        col.push_back(m.pos[j]);
-                        val.push_back(m.S(n, j));
-                    }
-                rowptr.push_back(int(col.size()));
-            }
-            DevBuf<int> drow, dcol;
-            DevBuf<double> dval;
-            drow.upload(rowptr);
-            dcol.upload(col);
-            dval.upload(val);
-            launch_extract(c->stream, d.field.p, d.t->total, P.nsys, P.NZ, drow.p, dcol.p, dval.p, 0, 0, c->km,
+            const VarDev &v = var_dev(*c, isys, ivar);
+            launch_extract(c->stream, d.field.p, d.t->total, P.nsys, P.NZ, v.rowptr.p, v.col.p, v.val.p, 0, 0, c->km,
                            c->spec.p, 0);
             zbwd(*c, c->spec.p, c->Fz.p, 1);
             launch_ybwd(c->stream, c->py, c->Fz.p, c->G.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
@@ -2283,22 +2368,12 @@ int coral_amd_set_variable_physical(coral_amd_ctx *c, int32_t kind, int32_t isys
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
-            const VarMaps m = var_maps(*d.t, P.NZ, ivar);
-            ensure_phys(*c);
-            std::vector<double> h(size_t(P.NXAA) * P.NYAA * P.NZAA);
-            for (int x = 0; x < P.NXAA; ++x)
-                for (int y = 0; y < P.NYAA; ++y)
-                    for (int z = 0; z < P.NZAA; ++z)
-                        h[(size_t(z) * P.NYAA + y) * P.NXAA + x] = in[(size_t(x) * P.NYAA + y) * P.NZAA + z];
-            HIP_OK(hipMemcpy(c->physd.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+            const VarDev &v = var_dev(*c, isys, ivar);
+            upload_phys(*c, in);
             launch_xfwd(c->stream, c->px, c->physd.p, c->H.p, 1, (long long)P.NZAA * P.NYAA, P.nkx);
             launch_yfwd(c->stream, c->py, c->H.p, c->Hy.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
             zfwd(*c, c->Hy.p, c->Qhat.p, 1);
-            DevBuf<double> dsinv;
-            DevBuf<int> dpos;
-            dsinv.upload(m.Sinv);
-            dpos.upload(m.pos);
-            launch_insert_var(c->stream, c->Qhat.p, P.nsys, m.ncol, dsinv.p, dpos.p, d.field.p, d.t->total);
+            launch_insert_var(c->stream, c->Qhat.p, P.nsys, v.ncol, v.Sinv.p, v.pos.p, d.field.p, d.t->total);
             HIP_OK(hipStreamSynchronize(c->stream));
         } else if (kind == 1) {
             if (isys < 0 || isys >= int(c->zs.size())) throw std::runtime_error("bad mean system index");
@@ -2409,29 +2484,14 @@ int coral_amd_products(coral_amd_ctx *c, double *out) {
         }
         c->side_advance = true;
         join_mean(*c);
-        HIP_OK(hipStreamSynchronize(c->stream));
-        std::vector<double2> h(size_t(P.nquad) * P.NZ * P.nsys);
-        if (fp32) {
-            std::vector<float2> hf(h.size());
-            HIP_OK(hipMemcpy(hf.data(), c->Qhat32.p, hf.size() * sizeof(float2), hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < h.size(); ++i) h[i] = make_double2(hf[i].x, hf[i].y);
-        } else {
-            HIP_OK(hipMemcpy(h.data(), c->Qhat.p, h.size() * sizeof(double2), hipMemcpyDeviceToHost));
-        }
-        // [q][ix][y slot][n], dealiased ky slots zero
-        const size_t per_q = size_t(P.nkx) * P.NYAA * P.NZ;
-        std::fill(out, out + 2 * per_q * P.nquad, 0.0);
-        for (int q = 0; q < P.nquad; ++q)
-            for (int ix = 0; ix < P.nkx; ++ix)
-                for (int jy = 0; jy < P.nky; ++jy) {
-                    const size_t sy = size_t(ix) * P.nky + jy;
-                    const size_t dst = size_t(q) * per_q + (size_t(ix) * P.NYAA + P.ky_slot[jy]) * P.NZ;
-                    for (int n = 0; n < P.NZ; ++n) {
-                        const double2 v = h[(size_t(q) * P.NZ + n) * P.nsys + sy];
-                        out[2 * (dst + n)] = v.x;
-                        out[2 * (dst + n) + 1] = v.y;
-                    }
-                }
+        // [q][n][s] -> [q][s][n] on the device, then [q][ix][y slot][n]
+        const size_t nsys = P.nsys, per = nsys * P.NZ;
+        ensure_hostd(*c, per * P.nquad);
+        if (fp32)
+            transpose(c->stream, c->Qhat32.p, P.NZ, P.nsys, nsys, per, c->hostd.p, P.NZ, per, P.nquad);
+        else
+            transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, nsys, per, c->hostd.p, P.NZ, per, P.nquad);
+        download_modes(*c, c->hostd.p, P.nquad, P.NZ, out);
         return 0;
     } catch (const std::exception &e) {
         return fail(e);
@@ -2444,15 +2504,9 @@ int coral_amd_bwd_transform(coral_amd_ctx *c, const double *spec, double *phys) 
         const Problem &P = c->P;
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        std::vector<double2> h(size_t(P.nsys) * P.NZ);
-        for (int ix = 0; ix < P.nkx; ++ix)
-            for (int jy = 0; jy < P.nky; ++jy) {
-                const size_t src = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * P.NZ;
-                const size_t sy = size_t(ix) * P.nky + jy;
-                for (int n = 0; n < P.NZ; ++n)
-                    h[size_t(n) * P.nsys + sy] = make_double2(spec[2 * (src + n)], spec[2 * (src + n) + 1]);
-            }
-        HIP_OK(hipMemcpy(c->spec.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
+        ensure_hostd(*c, size_t(P.nsys) * P.NZ);
+        upload_modes(*c, spec, P.NZ, c->hostd.p);
+        transpose(c->stream, c->hostd.p, P.nsys, P.NZ, P.NZ, 0, c->spec.p, P.nsys, 0, 1);
         zbwd(*c, c->spec.p, c->Fz.p, 1);
         launch_ybwd(c->stream, c->py, c->Fz.p, c->G.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
         const long long nlines = (long long)P.NZAA * P.NYAA;
@@ -2471,31 +2525,15 @@ int coral_amd_fwd_transform(coral_amd_ctx *c, const double *phys, double *spec) 
         const Problem &P = c->P;
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        ensure_phys(*c);
-        // host [x][y][z] -> device [z][y][x]
-        std::vector<double> h(size_t(P.NXAA) * P.NYAA * P.NZAA);
-        for (int x = 0; x < P.NXAA; ++x)
-            for (int y = 0; y < P.NYAA; ++y)
-                for (int z = 0; z < P.NZAA; ++z)
-                    h[(size_t(z) * P.NYAA + y) * P.NXAA + x] = phys[(size_t(x) * P.NYAA + y) * P.NZAA + z];
-        HIP_OK(hipMemcpy(c->physd.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+        upload_phys(*c, phys);
         const long long nlines = (long long)P.NZAA * P.NYAA;
         launch_xfwd(c->stream, c->px, c->physd.p, c->H.p, 1, nlines, P.nkx);
         launch_yfwd(c->stream, c->py, c->H.p, c->Hy.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
         zfwd(*c, c->Hy.p, c->Qhat.p, 1);
         HIP_OK(hipStreamSynchronize(c->stream));
-        std::vector<double2> q(size_t(P.nsys) * P.NZ);
-        HIP_OK(hipMemcpy(q.data(), c->Qhat.p, q.size() * sizeof(double2), hipMemcpyDeviceToHost));
-        std::memset(spec, 0, sizeof(double) * 2 * size_t(P.nkx) * P.NYAA * P.NZ);
-        for (int ix = 0; ix < P.nkx; ++ix)
-            for (int jy = 0; jy < P.nky; ++jy) {
-                const size_t dst = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * P.NZ;
-                const size_t sy = size_t(ix) * P.nky + jy;
-                for (int n = 0; n < P.NZ; ++n) {
-                    spec[2 * (dst + n)] = q[size_t(n) * P.nsys + sy].x;
-                    spec[2 * (dst + n) + 1] = q[size_t(n) * P.nsys + sy].y;
-                }
-            }
+        ensure_hostd(*c, size_t(P.nsys) * P.NZ);
+        transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, P.nsys, 0, c->hostd.p, P.NZ, 0, 1);
+        download_modes(*c, c->hostd.p, 1, P.NZ, spec);
         return 0;
     } catch (const std::exception &e) {
         return fail(e);
@@ -2606,29 +2644,11 @@ int coral_amd_system_solve(coral_amd_ctx *c, int32_t isys, const double *rhs, do
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
         HIP_OK(hipStreamSynchronize(c->side));
-        const Problem &P = c->P;
         SysDev &d = *c->ks[isys];
         const int total = d.t->total;
-        std::vector<double2> h(size_t(P.nsys) * total);
-        for (int ix = 0; ix < P.nkx; ++ix)
-            for (int jy = 0; jy < P.nky; ++jy) {
-                const size_t s = size_t(ix) * P.nky + jy, src = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * total;
-                for (int i = 0; i < total; ++i)
-                    h[s * total + i] = make_double2(rhs[2 * (src + i)], rhs[2 * (src + i) + 1]);
-            }
-        HIP_OK(hipMemcpy(d.R.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
+        upload_modes(*c, rhs, total, d.R.p);
         solve_system(*c, d, d.R.p, d.X[0]->p);
-        HIP_OK(hipStreamSynchronize(c->stream));
-        HIP_OK(hipMemcpy(h.data(), d.X[0]->p, h.size() * sizeof(double2), hipMemcpyDeviceToHost));
-        std::memset(x, 0, sizeof(double) * 2 * size_t(P.nkx) * P.NYAA * total);
-        for (int ix = 0; ix < P.nkx; ++ix)
-            for (int jy = 0; jy < P.nky; ++jy) {
-                const size_t s = size_t(ix) * P.nky + jy, dst = (size_t(ix) * P.NYAA + P.ky_slot[jy]) * total;
-                for (int i = 0; i < total; ++i) {
-                    x[2 * (dst + i)] = h[s * total + i].x;
-                    x[2 * (dst + i) + 1] = h[s * total + i].y;
-                }
-            }
+        download_modes(*c, d.X[0]->p, 1, total, x);
         return 0;
     } catch (const std::exception &e) {
         return fail(e);
