@@ -146,12 +146,14 @@ struct coral_amd_ctx {
     Problem P;
     int device = 0;
     hipStream_t stream = nullptr;
-    // the mean systems' NL terms, right-hand sides and solves run on a second
-    // stream, overlapped with the kxky work: they wait for Qhat (ev_qhat) and
-    // the kxky side waits for their solutions (ev_mean) before the next
-    // stage's mean extraction
-    hipStream_t side = nullptr;
-    hipEvent_t ev_qhat = nullptr, ev_mean = nullptr;
+    // the mean systems' NL terms, right-hand sides and solves run on side
+    // streams (mean system k on stream k mod NSIDE, so that their chains of
+    // small kernels run beside each other too), overlapped with the kxky work:
+    // they wait for Qhat (ev_qhat) and the kxky side waits for their solutions
+    // (ev_mean) before the next stage's mean extraction
+    static constexpr int NSIDE = 2;
+    hipStream_t side[NSIDE] = {};
+    hipEvent_t ev_qhat = nullptr, ev_mean[NSIDE] = {};
     bool mean_pending = false;
     KeptModes km{};
     std::vector<std::unique_ptr<SysDev>> ks, zs;
@@ -268,8 +270,10 @@ struct coral_amd_ctx {
         }
         drop_graphs();
         if (ev_qhat) (void)hipEventDestroy(ev_qhat);
-        if (ev_mean) (void)hipEventDestroy(ev_mean);
-        if (side) (void)hipStreamDestroy(side);
+        for (auto &e : ev_mean)
+            if (e) (void)hipEventDestroy(e);
+        for (auto &st : side)
+            if (st) (void)hipStreamDestroy(st);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -306,16 +310,6 @@ struct coral_amd_ctx {
 };
 
 namespace {
-
-// Clears the CFL maxima with a kernel rather than hipMemsetAsync, so that a
-// caller who captures the step into a HIP graph records no memset node.
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-void zero_cflmax(hipStream_t st, unsigned long long *p) {
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, p, 3);
-    check_launch("zero_cflmax");
-}
 
 FFTPlan make_plan(int N, DevBuf<double2> &tw) {
     FFTPlan p;
@@ -753,10 +747,11 @@ void nl_assemble(coral_amd_ctx &c, SysDev &d, double2 *Khat) {
     c.timed(d.kxky ? "nl_assemble" : "nl_mean", [&] { launch_nl(c.stream, a); });
 }
 
-// the main stream waits for the mean systems' pending work on the side stream
+// the main stream waits for the mean systems' pending work on the side streams
 void join_mean(coral_amd_ctx &c) {
     if (!c.mean_pending) return;
-    HIP_OK(hipStreamWaitEvent(c.stream, c.ev_mean, 0));
+    for (size_t k = 0; k < std::min<size_t>(c.zs.size(), c.NSIDE); ++k)
+        HIP_OK(hipStreamWaitEvent(c.stream, c.ev_mean[k], 0));
     c.mean_pending = false;
 }
 
@@ -772,24 +767,26 @@ void swap_step_buffers(coral_amd_ctx &c) {
     ++c.nswap;
 }
 
-// f's launches (and timer events) go to the side stream
+// f's launches (and timer events) go to side stream k
 template <class F>
-void on_side(coral_amd_ctx &c, F &&f) {
-    std::swap(c.stream, c.side);
+void on_side(coral_amd_ctx &c, int k, F &&f) {
+    std::swap(c.stream, c.side[k]);
     try {
         f();
     } catch (...) {
-        std::swap(c.stream, c.side);
+        std::swap(c.stream, c.side[k]);
         throw;
     }
-    std::swap(c.stream, c.side);
+    std::swap(c.stream, c.side[k]);
 }
 
 // Chebyshev coefficients of all full variables from the given states, then the
 // backward transforms up to G.
-// fp32: the FP32 chain into spec32 / Fz32 / G32 (the step in precision mode 1)
+// fp32: the FP32 chain into spec32 / Fz32 / G32 (the step in precision mode 1);
+// clear_cfl: the CFL maxima cleared on the way (by a kernel rather than
+// hipMemsetAsync, so that a captured step records no memset node)
 void backward_to_G(coral_amd_ctx &c, const std::vector<const double2 *> &kst, const std::vector<const double2 *> &zst,
-                   bool fp32 = false) {
+                   bool fp32 = false, bool clear_cfl = false) {
     const Problem &P = c.P;
     const size_t fsz = size_t(P.nsys) * P.NZ;
     c.timed("extract", [&] {
@@ -823,15 +820,23 @@ void backward_to_G(coral_amd_ctx &c, const std::vector<const double2 *> &kst, co
         if (fp32) a.spec32 = c.spec32.p;
         if (P.nfull > 0) launch_extract_all(c.stream, a);
         join_mean(c);   // the mean states below come from the side stream
+        ExtractMeanArgs m{};
+        m.nfull = P.nfull;
+        m.NZ = P.NZ;
+        m.nsys = P.nsys;
+        m.spec = c.spec.p;
+        m.spec32 = fp32 ? c.spec32.p : nullptr;
+        m.clear = clear_cfl ? c.cflmax.p : nullptr;
         for (auto &e : c.ext) {
             if (e->kind != 1) continue;
-            if (fp32)
-                launch_extract_mean32(c.stream, zst[e->system], P.NZ, P.nsys, e->rowptr.p, e->col.p, e->val.p,
-                                      c.spec32.p + e->full * fsz);
-            else
-                launch_extract_mean(c.stream, zst[e->system], P.NZ, P.nsys, e->rowptr.p, e->col.p, e->val.p,
-                                    c.spec.p + e->full * fsz);
+            if (m.nterms == MAX_EXTRACT_TERMS) {
+                launch_extract_mean(c.stream, m);
+                m.nterms = 0;
+                m.clear = nullptr;
+            }
+            m.term[m.nterms++] = ExtractMeanTerm{e->rowptr.p, e->col.p, e->val.p, zst[e->system], e->full};
         }
+        if (m.nterms || m.clear) launch_extract_mean(c.stream, m);
         // boundary values and vertical decompositions of the full variables
         // (marching.f90:544-577), on their complete coefficients
         for (int f = 0; f < P.nfull && f < (int)c.full_filter.size(); ++f) {
@@ -1009,8 +1014,7 @@ void side_products(coral_amd_ctx &c) {
 void products_to_Qhat(coral_amd_ctx &c, const std::vector<const double2 *> &kst,
                       const std::vector<const double2 *> &zst, bool fp32 = false) {
     const Problem &P = c.P;
-    backward_to_G(c, kst, zst, fp32);
-    zero_cflmax(c.stream, c.cflmax.p);
+    backward_to_G(c, kst, zst, fp32, true);
     XPassArgs xa{};
     xa.G = fp32 ? reinterpret_cast<const double2 *>(c.G32.p) : c.G.p;
     xa.H = fp32 ? reinterpret_cast<double2 *>(c.H32.p) : c.H.p;
@@ -1511,13 +1515,6 @@ void nl_terms(coral_amd_ctx &c, const std::vector<const double2 *> &kst, const s
     if (!c.zs.empty()) HIP_OK(hipEventRecord(c.ev_qhat, c.stream));
 }
 
-// NL terms of the mean systems from the Qhat of nl_terms (on the stream they
-// are launched on, after ev_qhat)
-void nl_terms_mean(coral_amd_ctx &c, int stage) {
-    HIP_OK(hipStreamWaitEvent(c.stream, c.ev_qhat, 0));
-    for (auto &d : c.zs) nl_assemble(c, *d, d->Khat[stage]->p);
-}
-
 // (M - dt a11 L) out = rhs for every wavenumber of a system, with the factors
 // of the last set_dt (backsolve_to_aux, PL_IMEX_timestepping_marching.f90:57-58)
 // the 16-lane solve's arguments for system d (false: d uses another kernel)
@@ -1619,7 +1616,7 @@ void project_kx0(coral_amd_ctx &c) {
 // x^{n+1} = x_s.
 // A step in phases (one_step_beyond, PL_IMEX_timestepping_marching.f90:3-48):
 // step_begin (the stage coefficients), per stage stage_nl (NL terms, the mean
-// systems on the side stream) and per kxky system stage_rhs then
+// systems on the side streams) and per kxky system stage_rhs then
 // stage_solve, and step_end.  one_step runs them for one run; the ensemble's
 // lockstep step runs every run's stage_nl and stage_rhs, then their solves
 // as one launch.
@@ -1680,23 +1677,24 @@ void stage_solve(coral_amd_ctx &c, int i, SysDev &d) {
     if (c.refine == 2 || (c.refine == 1 && i == s - 1)) refine_solution(c, d, d.R.p, d.X[i]->p, c.P.a_arr[i * s + i]);
 }
 
-// stage i's NL terms, and the mean systems' whole stage on the side stream
+// stage i's NL terms, and the mean systems' whole stage on the side streams
 void stage_nl(coral_amd_ctx &c, int i) {
     std::vector<const double2 *> kst, zst;
     for (auto &d : c.ks) kst.push_back(i == 0 ? d->field.p : d->X[i - 1]->p);
     for (auto &d : c.zs) zst.push_back(i == 0 ? d->field.p : d->X[i - 1]->p);
     nl_terms(c, kst, zst, i);
-    if (!c.zs.empty()) {
-        on_side(c, [&] {
-            nl_terms_mean(c, i);
-            for (auto &d : c.zs) {
-                stage_rhs(c, i, *d);
-                stage_solve(c, i, *d);
-            }
-            HIP_OK(hipEventRecord(c.ev_mean, c.stream));
+    const int nz = int(c.zs.size());
+    for (int k = 0; k < nz; ++k)
+        on_side(c, k % c.NSIDE, [&] {
+            SysDev &d = *c.zs[k];
+            // NL terms from the Qhat of nl_terms
+            if (k < c.NSIDE) HIP_OK(hipStreamWaitEvent(c.stream, c.ev_qhat, 0));
+            nl_assemble(c, d, d.Khat[i]->p);
+            stage_rhs(c, i, d);
+            stage_solve(c, i, d);
+            if (k + c.NSIDE >= nz) HIP_OK(hipEventRecord(c.ev_mean[k % c.NSIDE], c.stream));
         });
-        c.mean_pending = true;
-    }
+    c.mean_pending = nz > 0;
 }
 
 void step_end(coral_amd_ctx &c) {
@@ -1717,8 +1715,8 @@ void one_step(coral_amd_ctx &c) {
     step_end(c);
 }
 
-// Two graphs of one step each, captured from the stream (the side stream
-// joins through its events).  Capturing runs one_step's host logic, which
+// Two graphs of one step each, captured from the stream (the side streams
+// join through their events).  Capturing runs one_step's host logic, which
 // swaps the step buffers; after both captures they are back where they were.
 // The step holds no memset and no allocation, so the graphs replay it
 // exactly; they are dropped when dt changes.
@@ -1895,9 +1893,9 @@ int coral_amd_create(const coral_amd_problem *prob, int device, coral_amd_ctx **
         c->device = device;
         HIP_OK(hipSetDevice(device));
         HIP_OK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-        HIP_OK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+        for (auto &st : c->side) HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
         HIP_OK(hipEventCreateWithFlags(&c->ev_qhat, hipEventDisableTiming));
-        HIP_OK(hipEventCreateWithFlags(&c->ev_mean, hipEventDisableTiming));
+        for (auto &e : c->ev_mean) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         c->km = KeptModes{P.nkx, P.nky, P.NY, P.kx_box, P.ky_box};
         for (auto &t : P.kxky) {
             c->ks.emplace_back(new SysDev());
@@ -2021,7 +2019,7 @@ int coral_amd_upload_state(coral_amd_ctx *c, int32_t kind, int32_t isys, const d
         // the copies below go through the null stream, which does not wait
         // for the context's non-blocking streams: finish queued steps first
         HIP_OK(hipStreamSynchronize(c->stream));
-        HIP_OK(hipStreamSynchronize(c->side));
+        for (auto &st : c->side) HIP_OK(hipStreamSynchronize(st));
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
@@ -2414,8 +2412,7 @@ int coral_amd_horizontal_averages(coral_amd_ctx *c, double *full_avg, double *qu
         col.alloc(size_t(nf) * P.NZ + size_t(nq) * P.NZAA);
         if (quad_avg) {
             // products of the current state up to the y transform; column s = 0 is the (0,0) mode
-            backward_to_G(*c, kst, zst);
-            zero_cflmax(c->stream, c->cflmax.p);
+            backward_to_G(*c, kst, zst, false, true);
             XPassArgs xa{};
             xa.G = c->G.p;
             xa.H = c->H.p;
@@ -2643,7 +2640,7 @@ int coral_amd_system_solve(coral_amd_ctx *c, int32_t isys, const double *rhs, do
         if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        HIP_OK(hipStreamSynchronize(c->side));
+        for (auto &st : c->side) HIP_OK(hipStreamSynchronize(st));
         SysDev &d = *c->ks[isys];
         const int total = d.t->total;
         upload_modes(*c, rhs, total, d.R.p);
@@ -2699,7 +2696,7 @@ int coral_amd_set_precision(coral_amd_ctx *c, int32_t mode, int32_t refine) {
             throw std::runtime_error("fixed physical fields and the Smagorinsky viscosity run with the FP64 transform chain only");
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        HIP_OK(hipStreamSynchronize(c->side));
+        for (auto &st : c->side) HIP_OK(hipStreamSynchronize(st));
         Problem &P = c->P;
         if (mode == 1 && !c->spec32.p) {
             ZFrags32 zf;
@@ -3369,7 +3366,7 @@ bool ens_lockstep_ok(const coral_amd_ensemble &e, std::string *why = nullptr) {
 }
 
 // The lockstep graphs (one per buffer assignment): per stage every run's NL
-// terms (its mean systems forked onto its side stream) and kxky right-hand
+// terms (its mean systems forked onto its side streams) and kxky right-hand
 // sides, then the stage's kxky solves grouped by kernel variant, each group
 // one k_solve16_batch launch; systems the 16-lane solve does not take are
 // solved on their own.  Every run's arithmetic is its own step's.

@@ -217,28 +217,31 @@ void launch_extract_all(hipStream_t st, const ExtractAllArgs &a) {
     CHECK_LAUNCH();
 }
 
-// mean contributions land in the (0,0) column: spec[n][0] (C = double2, or
-// float2 in the FP32 chain, where the FP64 sum is rounded once)
-template <class C>
-__global__ void k_extract_mean(const double2 *__restrict__ zstate, int NZ, int nsys, const int *__restrict__ rowptr,
-                               const int *__restrict__ col, const double *__restrict__ val, C *spec) {
-    for (int n = threadIdx.x; n < NZ; n += blockDim.x) {
+// mean contributions land in the (0,0) column: spec[n][0] (the FP32 chain
+// rounds after each term), one thread per (full variable, n).  One launch for
+// every term and for clearing the CFL maxima: as a launch each they were 11 of
+// 172 us per stage at 64 x 64 x 33, and a gap of 2 to 3 us before each.
+__global__ __launch_bounds__(256) void k_extract_mean(ExtractMeanArgs a) {
+    if (blockIdx.x == 0 && a.clear && threadIdx.x < 3) a.clear[threadIdx.x] = 0ull;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= a.nfull * a.NZ) return;
+    const int f = e / a.NZ, n = e - f * a.NZ;
+    for (int t = 0; t < a.nterms; ++t) {
+        const ExtractMeanTerm &T = a.term[t];
+        if (T.full != f) continue;
         double acc = 0.0;
-        for (int k = rowptr[n]; k < rowptr[n + 1]; ++k) acc += val[k] * zstate[col[k]].x;
-        C &o = spec[(size_t)n * nsys];
-        o.x = typename CxT<C>::R(double(o.x) + acc);
+        for (int k = T.rowptr[n]; k < T.rowptr[n + 1]; ++k) acc += T.val[k] * T.zstate[T.col[k]].x;
+        if (a.spec32) {
+            float2 &o = a.spec32[(size_t)e * a.nsys];
+            o.x = float(double(o.x) + acc);
+        } else {
+            a.spec[(size_t)e * a.nsys].x += acc;
+        }
     }
 }
 
-void launch_extract_mean(hipStream_t st, const double2 *zstate, int NZ, int nsys, const int *rowptr, const int *col,
-                         const double *val, double2 *spec) {
-    hipLaunchKernelGGL(k_extract_mean<double2>, dim3(1), dim3(256), 0, st, zstate, NZ, nsys, rowptr, col, val, spec);
-    CHECK_LAUNCH();
-}
-
-void launch_extract_mean32(hipStream_t st, const double2 *zstate, int NZ, int nsys, const int *rowptr, const int *col,
-                           const double *val, float2 *spec) {
-    hipLaunchKernelGGL(k_extract_mean<float2>, dim3(1), dim3(256), 0, st, zstate, NZ, nsys, rowptr, col, val, spec);
+void launch_extract_mean(hipStream_t st, const ExtractMeanArgs &a) {
+    hipLaunchKernelGGL(k_extract_mean, dim3(std::max(1u, blocks_for(a.nfull * a.NZ, 256))), dim3(256), 0, st, a);
     CHECK_LAUNCH();
 }
 
@@ -2105,7 +2108,7 @@ __global__ __launch_bounds__(64) void k_solve16_batch(const Solve16Args *__restr
 }
 
 bool solve16_shape(const Solve16Args &a, Solve16Shape &sh) {
-    if (a.kl > 16 || a.n < 32 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol || !a.sink) return false;
+    if (a.kl > 16 || a.n < 1 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol || !a.sink) return false;
     if (a.nslot < 1 || a.nslot > SOLVE16_SLOTS || (a.nslot > 1 && !a.mem)) return false;
     sh.nq = 1 + (a.kv + 15) / 16;
     if (sh.nq < 2 || sh.nq > 4) return false;
@@ -2239,7 +2242,7 @@ void solve16_trim_u_copy(hipStream_t st, const void *Ufull, int elem, int n, int
 
 int solve16_ncol(int n, int kl, int kv) {
     // (positions are packed in 14 bits of the position words)
-    if (kl > 16 || n < 32 || n >= SOLVE16_NONE || 1 + (kv + 15) / 16 > 4) return 0;
+    if (kl > 16 || n < 1 || (n < 32 && kv < 1) || n >= SOLVE16_NONE || 1 + (kv + 15) / 16 > 4) return 0;
     return 16 * ((n + 15) / 16 + 1);
 }
 

@@ -40,11 +40,23 @@ struct ExtractAllArgs {
     int stotal[MAX_EXTRACT_STATES];
 };
 void launch_extract_all(hipStream_t st, const ExtractAllArgs &a);
-// mean contributions into the (0,0) column: spec[n][0] += sum val[k] * Re(zstate[col[k]])
-void launch_extract_mean(hipStream_t st, const double2 *zstate, int NZ, int nsys, const int *rowptr, const int *col,
-                         const double *val, double2 *spec);
-void launch_extract_mean32(hipStream_t st, const double2 *zstate, int NZ, int nsys, const int *rowptr, const int *col,
-                           const double *val, float2 *spec);
+// mean contributions of all terms into the (0,0) columns, spec[full][n][0] +=
+// sum val[k] * Re(zstate[col[k]]) term after term, into spec32 when set; clear:
+// three words to zero on the way (null: none)
+struct ExtractMeanTerm {
+    const int *rowptr, *col;
+    const double *val;
+    const double2 *zstate;
+    int full;
+};
+struct ExtractMeanArgs {
+    int nterms, nfull, NZ, nsys;
+    ExtractMeanTerm term[MAX_EXTRACT_TERMS];
+    double2 *spec;
+    float2 *spec32;
+    unsigned long long *clear;
+};
+void launch_extract_mean(hipStream_t st, const ExtractMeanArgs &a);
 
 // ---- z transforms ----
 // Layouts (z-major): spec[b][n][s], Fz[b][z][s], Hy[b][z][s], Qhat[b][n][s] (complex s)
