@@ -1793,8 +1793,8 @@ void download_phys(coral_amd_ctx &c, double *out) {
     double *d = reinterpret_cast<double *>(c.hostd.p);
     const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
     transpose(c.stream, c.physd.p, P.NZAA, P.NXAA, NY * NX, NX, d, NY * NZ, NZ, P.NYAA);
-    c.host.to_host(c.stream, c.device, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return out + x * NY * NZ; },
-                   [](int, int) {});
+    c.host.to_host(c.stream, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return out + x * NY * NZ; },
+                   [](size_t, size_t) {});
 }
 
 // host [x][y][z] -> device [z][y][x]
@@ -1804,7 +1804,7 @@ void upload_phys(coral_amd_ctx &c, const double *in) {
     ensure_hostd(c, (c.physd.n + 1) / 2);
     double *d = reinterpret_cast<double *>(c.hostd.p);
     const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
-    c.host.to_device(c.stream, c.device, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return in + x * NY * NZ; });
+    c.host.to_device(c.stream, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return in + x * NY * NZ; });
     transpose(c.stream, d, P.NXAA, P.NZAA, NY * NZ, NZ, c.physd.p, NY * NX, NX, P.NYAA);
 }
 
@@ -1815,12 +1815,12 @@ void download_modes(coral_amd_ctx &c, const double2 *dev, int nf, int nv, double
     const size_t nsys = P.nsys, row = size_t(nv) * sizeof(double2), line = size_t(P.NYAA) * row;
     char *o = reinterpret_cast<char *>(out);
     c.host.to_host(
-        c.stream, c.device, dev, nf * nsys, row,
+        c.stream, dev, nf * nsys, row,
         [&](size_t r) {
             const size_t f = r / nsys, s = r - f * nsys, ix = s / P.nky, jy = s - ix * P.nky;
             return o + (f * P.nkx + ix) * line + P.ky_slot[jy] * row;
         },
-        [&](int part, int parts) {
+        [&](size_t part, size_t parts) {
             // the dealiased slots of a line follow the non-negative ky
             for (size_t l = part; l < size_t(nf) * P.nkx; l += parts)
                 std::memset(o + l * line + (P.NY / 2) * row, 0, (P.NYAA - P.nky) * row);
@@ -1832,7 +1832,7 @@ void upload_modes(coral_amd_ctx &c, const double *in, int nv, double2 *dev) {
     const Problem &P = c.P;
     const size_t row = size_t(nv) * sizeof(double2), line = size_t(P.NYAA) * row;
     const char *h = reinterpret_cast<const char *>(in);
-    c.host.to_device(c.stream, c.device, dev, P.nsys, row, [&](size_t s) {
+    c.host.to_device(c.stream, dev, P.nsys, row, [&](size_t s) {
         const size_t ix = s / P.nky, jy = s - ix * P.nky;
         return h + ix * line + P.ky_slot[jy] * row;
     });
