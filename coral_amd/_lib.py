@@ -83,7 +83,7 @@ EXPORTS = (
     "coral_amd_set_full_variable_filter", "coral_amd_add_source_term", "coral_amd_clear_source_terms",
     "coral_amd_set_source", "coral_amd_set_fixed_physical", "coral_amd_set_smagorinsky", "coral_amd_nn_mode_scale_t", "coral_amd_nn_modes_supported",
     "coral_amd_nn_modes_work", "coral_amd_nn_modes", "coral_amd_nn_tile_transpose",
-    "coral_amd_nn_gemm_bias",
+    "coral_amd_nn_gemm_bias", "coral_amd_nn_gemm16", "coral_amd_nn_gemm_gelu_bwd",
 )
 
 

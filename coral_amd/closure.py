@@ -60,6 +60,10 @@ def _bind():
     sig = {
         "coral_amd_nn_gemm": [c_int32, c_int32, c_int32, c_int32, c_int32, c_float, P, c_int32, c_int64, P, c_int32,
                               c_int64, c_float, P, c_int32, c_int64, c_int32, P, c_int64, P],
+        "coral_amd_nn_gemm16": [c_int32, c_int32, c_int32, c_int32, c_int32, c_float, P, c_int32, c_int64, P, c_int32,
+                                c_int64, c_float, P, c_int32, c_int64, c_int32, P, c_int64, P, P],
+        "coral_amd_nn_gemm_gelu_bwd_work": [c_int32, c_int32],
+        "coral_amd_nn_gemm_gelu_bwd": [c_int32, c_int32, c_int32, P, c_int32, P, c_int32, P, P, P, P, c_int64, P],
         "coral_amd_nn_gemm_work": [c_int32, c_int32, c_int32, c_int32],
         "coral_amd_nn_transpose_bf16": [P, c_int32, c_int32, P, P],
         "coral_amd_nn_mlp": [c_int64, c_int32, c_int32, P, P, P, P, P, P, P, P, P, P, P, c_int32, c_int32, P, P],
@@ -257,13 +261,14 @@ class _Work:
         self.part = DevArray(int(lib.coral_amd_nn_mse_partials(R * L.cout)))
         self.dH = DevArray(R * W)
         self.dH16 = DevArray(R * W, "bf16")
-        self.dA = DevArray(R * Hd)
         self.dZ16 = DevArray(R * Hd, "bf16")
         self.dCs = DevArray(P * nb * W)
         self.dCm16 = DevArray(P * nb * W, "bf16")
         self.wpart = DevArray(P * max(Hd * W, L.cin * W, W * L.cout))
-        self.work = DevArray(max(int(lib.coral_amd_nn_colsum_work(R, max(Hd, W, L.cout))),
+        self.work = DevArray(max(int(lib.coral_amd_nn_colsum_work(R, max(W, L.cout))),
                                  int(lib.coral_amd_nn_colsum_work(P, Hd * W))))
+        self.ngbwork = int(lib.coral_amd_nn_gemm_gelu_bwd_work(R, Hd))
+        self.gbwork = DevArray(self.ngbwork)
         # split-K partials of the long-K products (mode projections and the
         # per-plane weight gradients)
         shapes = [(nb, W, N2, P), (W, L.cout, N2, P), (Hd, W, N2, P), (W, Hd, N2, P), (L.cin, W, N2, P)]
@@ -327,10 +332,11 @@ class ClosureNet:
     def _p(self, name, t):
         return t.at(self.off[name][0])
 
-    def _gemm(self, tA, tB, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, batch=1, beta=0.0, alpha=1.0, ws=None):
+    def _gemm(self, tA, tB, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, batch=1, beta=0.0, alpha=1.0, ws=None,
+              C16=None):
         gw, ngw = (ws.gwork.ptr, ws.ngwork) if ws is not None else (None, 0)
-        check(lib.coral_amd_nn_gemm(tA, tB, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, gw, ngw,
-                                    None), "nn gemm")
+        check(lib.coral_amd_nn_gemm16(tA, tB, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, gw, ngw,
+                                      C16, None), "nn gemm")
 
     def _wt(self, l):
         """Device pointers of W1^T (hidden x width) and W2^T (width x hidden) of layer l."""
@@ -430,17 +436,17 @@ class ClosureNet:
         # projection
         self._wgrad(ws.H16[L.layers], W, ws.dY16, L.cout, W, L.cout, ws, self._p("Wp", g))
         colsum(ws.dY, L.cout, "bp")
-        self._gemm(0, 1, R, W, L.cout, ws.dY16.ptr, L.cout, 0, self._p("Wp", self.w16), L.cout, 0, ws.dH.ptr, W, 0)
+        self._gemm(0, 1, R, W, L.cout, ws.dY16.ptr, L.cout, 0, self._p("Wp", self.w16), L.cout, 0, ws.dH.ptr, W, 0,
+                   C16=ws.dH16.ptr)
         for l in reversed(range(L.layers)):
-            self._cast(ws.dH, ws.dH16)
             # MLP branch
             self._wgrad(ws.A16[l], Hd, ws.dH16, W, Hd, W, ws, self._p(f"W2.{l}", g))
             colsum(ws.dH, W, f"b2.{l}")
-            self._gemm(0, 1, R, Hd, W, ws.dH16.ptr, W, 0, self._p(f"W2.{l}", self.w16), W, 0, ws.dA.ptr, Hd, 0)
-            check(lib.coral_amd_nn_gelu_bwd(ws.Z[l].ptr, ws.dA.ptr, ws.dA.ptr, ws.dZ16.ptr, R * Hd, None),
-                  "nn gelu bwd")
+            # dZ = (dH W2^T) gelu'(Z) and db1, its column sums
+            check(lib.coral_amd_nn_gemm_gelu_bwd(R, Hd, W, ws.dH16.ptr, W, self._p(f"W2.{l}", self.w16), W,
+                                                 ws.Z[l].ptr, ws.dZ16.ptr, self._p(f"b1.{l}", g), ws.gbwork.ptr,
+                                                 ws.ngbwork, None), "nn gemm gelu bwd")
             self._wgrad(ws.H16[l], W, ws.dZ16, Hd, W, Hd, ws, self._p(f"W1.{l}", g))
-            colsum(ws.dA, Hd, f"b1.{l}")
             # spectral branch: dCs = B^T dH per plane; dD = sum_p Cm dCs; dCm = dCs D
             self._gemm(0, 0, nb, W, N2, self.basisT16.ptr, N2, 0, ws.dH16.ptr, W, N2 * W, ws.dCs.ptr, W, nb * W,
                        batch=P, ws=ws)
@@ -452,8 +458,7 @@ class ClosureNet:
             self._gemm(0, 1, R, W, Hd, ws.dZ16.ptr, Hd, 0, self._p(f"W1.{l}", self.w16), Hd, 0, ws.dH.ptr, W, 0,
                        beta=1.0)
             self._gemm(1, 0, N2, W, nb, self.basisT16.ptr, N2, 0, ws.dCm16.ptr, W, nb * W, ws.dH.ptr, W, N2 * W,
-                       batch=P, beta=1.0)
-        self._cast(ws.dH, ws.dH16)
+                       batch=P, beta=1.0, C16=ws.dH16.ptr)
         self._wgrad(X16, L.cin, ws.dH16, W, L.cin, W, ws, self._p("W0", g))
         colsum(ws.dH, W, "b0")
 

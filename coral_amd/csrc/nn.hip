@@ -40,13 +40,21 @@ __device__ inline unsigned short f2bf(float f) { return __builtin_bit_cast(unsig
 // ---------------------------------------------------------------------------
 constexpr int TM = 64, TN = 64, TK = 32, LDK = TK + 8;   // LDS row stride in bf16 (80 B)
 
-// Optional epilogue of an unsplit, unbatched product: C += bias (per
-// column), C16 = bf16(C) (same layout), C16T = bf16(C) in the tiled
-// transposed layout of tile_transpose (M % 32 == 0).
+// Optional epilogue of an unsplit product: C += bias (per column), C16 =
+// bf16(C) (same layout), C16T = bf16(C) in the tiled transposed layout of
+// tile_transpose (M % 32 == 0; the last two unbatched or C contiguous).
+// GELU (bound by memory: 147456 x 256 x 64 took 55 us as a product, 105 as
+// gelu_bwd and 31 as column sums, and takes 97 + 9 without the FP32 gradient in
+// memory): instead of C, with g = C * gelu'(Z) (Z in C's layout), C16 = bf16(g) and
+// part[row tile][column] = the sums of g over the tile's rows.
 struct GemmEpi {
     const float *bias = nullptr;
     unsigned short *C16 = nullptr, *C16T = nullptr;
+    const float *Z = nullptr;
+    float *part = nullptr;
 };
+__device__ inline float gelu_grad(float z);
+template <bool GELU>
 __global__ __launch_bounds__(256) void k_gemm_bf16(int transA, int transB, int M, int N, int K, float alpha,
                                                    const unsigned short *__restrict__ A, int lda, long long sA,
                                                    const unsigned short *__restrict__ B, int ldb, long long sB,
@@ -67,6 +75,32 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int transA, int transB, int M
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    // The products are formed as C^T = op(B)^T op(A)^T, so that a lane holds four
+    // consecutive columns of a row: result element q of tile (i, j) is row
+    // m0 + wm + 16 i + l % 16, column n0 + wn + 16 j + 4 (l / 16) + q.
+    const int rl = lane & 15, cq = 4 * (lane >> 4);
+    unsigned short *const C16 = epi.C16 ? epi.C16 + blockIdx.z * sC : nullptr;
+    // four columns at once where they are inside and 16-byte aligned
+    const bool vec = N % 4 == 0 && ldc % 4 == 0 && ((reinterpret_cast<uintptr_t>(GELU ? epi.Z : C) & 15) == 0) &&
+                     ((reinterpret_cast<uintptr_t>(C16) & 7) == 0);
+    f4 z[2][2];
+    if constexpr (GELU) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int gm = m0 + wm + 16 * i + rl, gn = n0 + wn + 16 * j + cq;
+                const float *p = epi.Z + (size_t)gm * ldc + gn;
+                z[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+                if (vec) {
+                    if (gm < M && gn < N) z[i][j] = *reinterpret_cast<const f4 *>(p);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (gm < M && gn + q < N) z[i][j][q] = p[q];
+                }
+            }
+    }
     // each operand's 64 x 32 slice is 256 vectors of 8 consecutive elements
     // along its contiguous dimension, one per thread; a vector inside the
     // matrix with a 16-byte aligned address is one load, others element by
@@ -146,35 +180,81 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int transA, int transB, int M
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
         __syncthreads();
     }
-    const int col = lane & 15, rq = 4 * (lane >> 4);
+    float cs[2][4] = {};   // column sums over the lane's rows (GELU)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int gm = m0 + wm + 16 * i + rl, gn = n0 + wn + 16 * j + cq;
+            if (gm >= M || gn >= N) continue;
+            const size_t o = (size_t)gm * ldc + gn;
+            f4 v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = alpha * acc[i][j][q];
+            if constexpr (GELU) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    v[q] = v[q] * gelu_grad(z[i][j][q]);
+                    if (gn + q < N) cs[j][q] += v[q];
+                }
+            } else if (vec) {
+                f4 *p = reinterpret_cast<f4 *>(C + o);
+                if (beta != 0.f) {
+                    const f4 c = *p;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = v[q] + beta * c[q];
+                }
+                if (epi.bias)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = v[q] + epi.bias[gn + q];
+                *p = v;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (gn + q < N) {
+                        if (beta != 0.f) v[q] = v[q] + beta * C[o + q];
+                        if (epi.bias) v[q] = v[q] + epi.bias[gn + q];
+                        C[o + q] = v[q];
+                    }
+            }
+            if (C16) {
+                unsigned short *h = C16 + o;
+                if (vec) {
+                    *reinterpret_cast<ushort4 *>(h) = make_ushort4(f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3]));
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (gn + q < N) h[q] = f2bf(v[q]);
+                }
+            }
+            if (epi.C16T)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (gn + q < N) epi.C16T[((size_t)(gm / 32) * N + gn + q) * 32 + (gm & 31)] = f2bf(v[q]);
+        }
+    if constexpr (GELU) {
+        // over the 16 rows of a lane group, then the two wavefronts of a column
+        float *sum = reinterpret_cast<float *>(As);   // [row half][column of the tile]
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int gm = m0 + wm + 16 * i + rq + q, gn = n0 + wn + 16 * j + col;
-                if (gm < M && gn < N) {
-                    float *p = C + (size_t)gm * ldc + gn;
-                    const float v0 = alpha * acc[i][j][q];
-                    float v = beta == 0.f ? v0 : v0 + beta * *p;
-                    if (epi.bias) v = v + epi.bias[gn];
-                    *p = v;
-                    if (epi.C16 || epi.C16T) {
-                        const unsigned short h = f2bf(v);
-                        if (epi.C16) epi.C16[(size_t)gm * ldc + gn] = h;
-                        if (epi.C16T) epi.C16T[((size_t)(gm / 32) * N + gn) * 32 + (gm & 31)] = h;
-                    }
-                }
+                float t = cs[j][q];
+                for (int d = 1; d < 16; d *= 2) t += __shfl_xor(t, d);
+                if (rl == 0) sum[(wv >> 1) * TN + wn + 16 * j + cq + q] = t;
             }
+        __syncthreads();
+        if (tid < TN && n0 + tid < N) epi.part[(size_t)blockIdx.y * N + n0 + tid] = sum[tid] + sum[TN + tid];
+    }
 }
 
 // C[b][m][n] = alpha sum_s P[b nsplit + s][m][n] + beta C[b][m][n]
 __global__ void k_splitk_sum(const float *__restrict__ P, int nsplit, int M, int N, int batch, float alpha,
-                             float beta, float *__restrict__ C, int ldc, long long sC) {
+                             float beta, float *__restrict__ C, int ldc, long long sC,
+                             unsigned short *__restrict__ C16) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x, mn = (long long)M * N;
     if (i >= mn * batch) return;
     const long long b = i / mn, e = i - b * mn;
@@ -182,9 +262,11 @@ __global__ void k_splitk_sum(const float *__restrict__ P, int nsplit, int M, int
     const float *p = P + b * nsplit * mn + e;
     float acc = 0.f;
     for (int s = 0; s < nsplit; ++s) acc += p[s * mn];
-    float *c = C + b * sC + (long long)m * ldc + n;
-    const float v = alpha * acc;
-    *c = beta == 0.f ? v : v + beta * *c;
+    const long long o = b * sC + (long long)m * ldc + n;
+    float v = alpha * acc;
+    if (beta != 0.f) v = v + beta * C[o];
+    C[o] = v;
+    if (C16) C16[o] = f2bf(v);
 }
 
 // Split of K for products with few output tiles and a long K (per-plane
@@ -210,7 +292,7 @@ long long gemm_work(int M, int N, int K, int batch) {
 
 void gemm(hipStream_t st, int transA, int transB, int M, int N, int K, float alpha, const unsigned short *A, int lda,
           long long sA, const unsigned short *B, int ldb, long long sB, float beta, float *C, int ldc, long long sC,
-          int batch, float *work, long long nwork) {
+          int batch, float *work, long long nwork, unsigned short *C16) {
     if (M <= 0 || N <= 0 || batch <= 0) return;
     if (K <= 0) throw std::runtime_error("gemm: K must be positive");
     int ns, kc;
@@ -218,19 +300,21 @@ void gemm(hipStream_t st, int transA, int transB, int M, int N, int K, float alp
     const dim3 grid(unsigned((N + TN - 1) / TN), unsigned((M + TM - 1) / TM), unsigned(batch * ns));
     if (grid.y > 65535u || (long long)batch * ns > 65535) throw std::runtime_error("gemm: grid too large (M or batch)");
     if (ns == 1) {
-        hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, st, transA, transB, M, N, K, alpha, A, lda, sA, B, ldb,
-                           sB, beta, C, ldc, sC, K, 1, GemmEpi{});
+        GemmEpi e;
+        e.C16 = C16;
+        hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, st, transA, transB, M, N, K, alpha, A, lda, sA, B,
+                           ldb, sB, beta, C, ldc, sC, K, 1, e);
         check_launch("bf16 gemm");
         return;
     }
     const long long need = (long long)ns * batch * M * N;
     if (!work || nwork < need)
         throw std::runtime_error("gemm: split-K work space of " + std::to_string(need) + " floats required");
-    hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, st, transA, transB, M, N, K, 1.f, A, lda, sA, B, ldb, sB, 0.f,
-                       work, N, (long long)M * N, kc, ns, GemmEpi{});
+    hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, st, transA, transB, M, N, K, 1.f, A, lda, sA, B, ldb, sB,
+                       0.f, work, N, (long long)M * N, kc, ns, GemmEpi{});
     const long long n = (long long)batch * M * N;
     hipLaunchKernelGGL(k_splitk_sum, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, work, ns, M, N, batch, alpha,
-                       beta, C, ldc, sC);
+                       beta, C, ldc, sC, C16);
     check_launch("bf16 gemm (split K)");
 }
 
@@ -248,9 +332,33 @@ void gemm_bias(hipStream_t st, int M, int N, int K, const unsigned short *A, int
     e.bias = bias;
     e.C16 = C16;
     e.C16T = C16T;
-    hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, st, 0, 0, M, N, K, 1.f, A, lda, 0LL, B, ldb, 0LL, 0.f, C, N,
+    hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, st, 0, 0, M, N, K, 1.f, A, lda, 0LL, B, ldb, 0LL, 0.f, C, N,
                        0LL, K, 1, e);
     check_launch("bf16 gemm + bias");
+}
+
+// dZ = (A B^T) * gelu'(Z) (A M x K, B N x K; Z M x N), dZ16 = bf16(dZ), out =
+// the column sums of dZ: gemm, gelu_bwd and colsum without the FP32 dZ in memory
+long long gemm_gelu_bwd_work(int M, int N) {
+    if (M <= 0 || N <= 0) return 0;
+    const long long nt = (M + TM - 1) / TM;
+    return nt * N + colsum_work(nt, N);
+}
+void gemm_gelu_bwd(hipStream_t st, int M, int N, int K, const unsigned short *A, int lda, const unsigned short *B,
+                   int ldb, const float *Z, unsigned short *dZ16, float *out, float *work, long long nwork) {
+    if (M <= 0 || N <= 0) return;
+    if (K <= 0) throw std::runtime_error("gemm: K must be positive");
+    if (!work || nwork < gemm_gelu_bwd_work(M, N)) throw std::runtime_error("gemm: work space for the column sums required");
+    const dim3 grid(unsigned((N + TN - 1) / TN), unsigned((M + TM - 1) / TM), 1);
+    if (grid.y > 65535u) throw std::runtime_error("gemm: grid too large (M)");
+    GemmEpi e;
+    e.C16 = dZ16;
+    e.Z = Z;
+    e.part = work;
+    hipLaunchKernelGGL(k_gemm_bf16<true>, grid, dim3(256), 0, st, 0, 1, M, N, K, 1.f, A, lda, 0LL, B, ldb, 0LL, 0.f,
+                       nullptr, N, 0LL, K, 1, e);
+    check_launch("bf16 gemm + gelu backward");
+    colsum(st, work, grid.y, N, out, work + (long long)grid.y * N, 0.f);
 }
 
 // dst (cols x rows) = src (rows x cols)^T, BF16 (the MLP kernel's weight
@@ -944,7 +1052,7 @@ void gelu_bwd(hipStream_t st, const float *z, const float *da, float *dz, unsign
 // are in flight), LDS adds the threads of a column.  One thread per column
 // and row chunk, then one per column over all chunks, left most of the chip
 // idle behind serial chains: they were 0.84 + 1.3 ms of the 4.94 ms of a
-// training step over 65536 points (width 64, hidden 256); it takes 3.04 ms now.
+// training step over 147456 points (width 64, hidden 256) and are 0.15 of 2.5.
 // Up to 256 rows are one chunk and one launch.
 template <int CW>
 __global__ __launch_bounds__(256) void k_colsum(const float *__restrict__ x, long long nrow, int chunk, int ncol,
@@ -1211,6 +1319,19 @@ int coral_amd_nn_gemm(int32_t transA, int32_t transB, int32_t M, int32_t N, int3
                       int32_t ldc, int64_t sC, int32_t batch, float *work, int64_t nwork, void *stream) {
     NN_ABI(coral::nn::gemm((hipStream_t)stream, transA, transB, M, N, K, alpha, (const unsigned short *)A, lda, sA,
                            (const unsigned short *)B, ldb, sB, beta, C, ldc, sC, batch, work, nwork))
+}
+int coral_amd_nn_gemm16(int32_t transA, int32_t transB, int32_t M, int32_t N, int32_t K, float alpha, const void *A,
+                        int32_t lda, int64_t sA, const void *B, int32_t ldb, int64_t sB, float beta, float *C,
+                        int32_t ldc, int64_t sC, int32_t batch, float *work, int64_t nwork, void *C16, void *stream) {
+    NN_ABI(coral::nn::gemm((hipStream_t)stream, transA, transB, M, N, K, alpha, (const unsigned short *)A, lda, sA,
+                           (const unsigned short *)B, ldb, sB, beta, C, ldc, sC, batch, work, nwork,
+                           (unsigned short *)C16))
+}
+int64_t coral_amd_nn_gemm_gelu_bwd_work(int32_t M, int32_t N) { return coral::nn::gemm_gelu_bwd_work(M, N); }
+int coral_amd_nn_gemm_gelu_bwd(int32_t M, int32_t N, int32_t K, const void *A, int32_t lda, const void *B, int32_t ldb,
+                               const float *Z, void *dZ16, float *out, float *work, int64_t nwork, void *stream) {
+    NN_ABI(coral::nn::gemm_gelu_bwd((hipStream_t)stream, M, N, K, (const unsigned short *)A, lda,
+                                    (const unsigned short *)B, ldb, Z, (unsigned short *)dZ16, out, work, nwork))
 }
 int64_t coral_amd_nn_gemm_work(int32_t M, int32_t N, int32_t K, int32_t batch) {
     return coral::nn::gemm_work(M, N, K, batch);

@@ -13,10 +13,16 @@ namespace nn {
 // transA), op(B) K x N (B is K x N, or N x K when transB), C FP32 M x N.
 // Products with few output tiles and a long K are split along K into
 // partials in work (gemm_work(M, N, K, batch) floats; throws if smaller).
+// C16 (optional, C's layout): bf16(C).
 void gemm(hipStream_t st, int transA, int transB, int M, int N, int K, float alpha, const unsigned short *A, int lda,
           long long sA, const unsigned short *B, int ldb, long long sB, float beta, float *C, int ldc, long long sC,
-          int batch, float *work = nullptr, long long nwork = 0);
+          int batch, float *work = nullptr, long long nwork = 0, unsigned short *C16 = nullptr);
 long long gemm_work(int M, int N, int K, int batch);
+// dZ = (A B^T) * gelu'(Z) (A M x K, B N x K, Z M x N): dZ16 = bf16(dZ), out [N] =
+// the column sums of dZ; work: gemm_gelu_bwd_work(M, N) floats
+void gemm_gelu_bwd(hipStream_t st, int M, int N, int K, const unsigned short *A, int lda, const unsigned short *B,
+                   int ldb, const float *Z, unsigned short *dZ16, float *out, float *work, long long nwork);
+long long gemm_gelu_bwd_work(int M, int N);
 // C (M x N) = A (M x K, lda) B (K x N, ldb) + bias, C16 = bf16(C), C16T =
 // bf16(C) tiled and transposed (tile_transpose's layout; M % 32 == 0), each
 // optional: the arithmetic of gemm, bias_act, tile_transpose

@@ -481,6 +481,16 @@ int coral_amd_nn_cast_bf16(const float *x, void *y, int64_t n, void *stream);
 int coral_amd_nn_bias_act(float *z, const float *bias, int32_t ncol, int64_t n, int32_t act, float *out, void *out16,
                           void *stream);
 int coral_amd_nn_gelu_bwd(const float *z, const float *da, float *dz, void *dz16, int64_t n, void *stream);
+/* coral_amd_nn_gemm with C16 = bf16(C) in C's layout as well (C16 may be null). */
+int coral_amd_nn_gemm16(int32_t transA, int32_t transB, int32_t M, int32_t N, int32_t K, float alpha, const void *A,
+                        int32_t lda, int64_t sA, const void *B, int32_t ldb, int64_t sB, float beta, float *C,
+                        int32_t ldc, int64_t sC, int32_t batch, float *work, int64_t nwork, void *C16, void *stream);
+/* coral_amd_nn_gemm (A M x K, B N x K transposed), _gelu_bwd and _colsum in one
+ * pass: dZ = (A B^T) * gelu'(Z), dZ16 = bf16(dZ), out[n] = sum_m dZ[m][n]; work:
+ * coral_amd_nn_gemm_gelu_bwd_work(M, N) floats. */
+int64_t coral_amd_nn_gemm_gelu_bwd_work(int32_t M, int32_t N);
+int coral_amd_nn_gemm_gelu_bwd(int32_t M, int32_t N, int32_t K, const void *A, int32_t lda, const void *B, int32_t ldb,
+                               const float *Z, void *dZ16, float *out, float *work, int64_t nwork, void *stream);
 /* column sums of x [nrow][ncol] into out (out = sums + beta out), deterministic;
  * work holds coral_amd_nn_colsum_work(nrow, ncol) floats */
 int64_t coral_amd_nn_colsum_work(int64_t nrow, int32_t ncol);
