@@ -1188,34 +1188,39 @@ typedef float cf4 __attribute__((ext_vector_type(4)));
 // FP32 -> BF16 with gfx950's conversion (as the network kernels' epilogues)
 __device__ inline unsigned short f2bf_hw(float f) { return __builtin_bit_cast(unsigned short, static_cast<__bf16>(f)); }
 
-// Rows per workgroup of the fused lift and projection: a tile lies inside one
-// x-line, so NXAA % LIFT_ROWS == 0 is required.
-constexpr int LIFT_ROWS = 64;
+// Rows per workgroup of the fused lift (a tile lies inside one x-line, 64 or 32
+// points; the tiled transposed copy is in blocks of 32 rows) and of the fused
+// projection.  Lines of 96, 288, ... points took the separate kernels before
+// tiles of 32: at 96 x 96 x 49 points, width 32, packing, lift, projection and
+// unpacking were 76 + 59 + 81 us, fused the two kernels take 101.
+int lift_rows(int NXAA) { return NXAA % 64 == 0 ? 64 : NXAA % 32 == 0 ? 32 : 0; }
+constexpr int PROJ_ROWS = 64;
 
 struct LiftShape {
     int kp = 0, ldk = 0;   // K rounded up to the MFMA depth; LDS row stride (bf16)
     size_t bytes = 0;      // dynamic LDS
 };
-LiftShape lift_shape(int nfull, int cin, int W) {
+LiftShape lift_shape(int nfull, int cin, int W, int rows) {
     LiftShape s;
     s.kp = (cin + 31) / 32 * 32;
     s.ldk = s.kp + 8;
-    // the input tile (bf16 [LIFT_ROWS][ldk]), later reused by the epilogue's
-    // FP32 tile [LIFT_ROWS][W + 4]
-    const size_t ops = sizeof(unsigned short) * size_t(LIFT_ROWS) * s.ldk;
-    const size_t epi = sizeof(float) * size_t(LIFT_ROWS) * (W + 4);
-    s.bytes = sizeof(double) * (size_t(9) * nfull * (LIFT_ROWS + 2) + 2 * size_t(s.kp)) + std::max(ops, epi);
+    // the input tile (bf16 [rows][ldk]), later reused by the epilogue's
+    // FP32 tile [rows][W + 4]
+    const size_t ops = sizeof(unsigned short) * size_t(rows) * s.ldk;
+    const size_t epi = sizeof(float) * size_t(rows) * (W + 4);
+    s.bytes = sizeof(double) * (size_t(9) * nfull * (rows + 2) + 2 * size_t(s.kp)) + std::max(ops, epi);
     return s;
 }
 
 // H = X W0 + b0 (FP32), H16 = bf16(H), H16T its tiled transposed copy (when
-// given), for LIFT_ROWS rows of the chunk at a time, X formed on chip: the
+// given), for LR rows of the chunk at a time, X formed on chip: the
 // input rows of k_closure_pack_lines (same values and rounding) are built in
 // LDS from the 3 x 3 neighbouring lines of every full variable and multiplied
 // on MFMA with the K order, zero padding and epilogue of nn::gemm_bias, so H,
 // H16 and H16T equal the pack-then-GEMM sequence's bit for bit without the
-// input rows ever reaching HBM.  One wavefront per 16 rows, all W columns.
-template <int W>
+// input rows ever reaching HBM.  A wavefront takes 16 rows and all W columns (64
+// rows) or half of them (32 rows).
+template <int W, int LR>
 __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__ phys,
                                                       const double *__restrict__ zgrid, int z0, int NXAA, int NYAA,
                                                       int NZAA, int nfull, int cin, int kp, int ldk,
@@ -1225,7 +1230,8 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
                                                       unsigned short *__restrict__ H16,
                                                       unsigned short *__restrict__ H16T) {
     extern __shared__ __align__(16) unsigned char lds[];
-    constexpr int LR = LIFT_ROWS, NT = W / 16, span = LR + 2;
+    constexpr int RG = LR / 16, NT = W / 16 * RG / 4, span = LR + 2;   // row groups; 16-column tiles of a wavefront
+    static_assert(LR == 32 || LR == 64, "a wavefront loads one or two lines at a time");
     const int N2 = NXAA * NYAA, ncore = 27 * nfull, ntile = 9 * nfull * span;
     double *tile = reinterpret_cast<double *>(lds);   // [dz][dy][f][x0-1 .. x0+LR]
     double *mv = tile + ntile, *rv = mv + kp;
@@ -1234,6 +1240,7 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
     const int zl = int(r0 / N2), rem = int(r0 - (long long)zl * N2), y = rem / NXAA, x0 = rem - y * NXAA;
     const int z = z0 + zl, tid = threadIdx.x;
     const int lane = tid & 63, wv = tid >> 6, fr = lane & 15, fk = 8 * (lane >> 4), rq = 4 * (lane >> 4);
+    const int wr = 16 * (wv % RG), wc = 16 * NT * (wv / RG);   // the wavefront's rows and columns
     // the B fragments (W0^T rows, zero past cin) straight from memory, issued first
     constexpr int KMAX = 8;   // kp <= 256
     cbf8 bfr[KMAX][NT];
@@ -1241,22 +1248,24 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
     for (int k = 0; k < KMAX; ++k)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-            if (32 * k < kp) bfr[k][j] = *reinterpret_cast<const cbf8 *>(W0T + (size_t)(16 * j + fr) * kp + 32 * k + fk);
-    // the neighbouring lines: wavefront wv takes lines wv, wv + 4, ... (line
-    // L = o nfull + f, o = 3 (dz+1) + (dy+1)), a lane the points lane and 64 +
-    // lane of the line's span; up to four lines' loads in flight before their
-    // LDS stores
+            if (32 * k < kp) bfr[k][j] = *reinterpret_cast<const cbf8 *>(W0T + (size_t)(wc + 16 * j + fr) * kp + 32 * k + fk);
+    // the neighbouring lines (line L = o nfull + f, o = 3 (dz+1) + (dy+1)): LR
+    // lanes per line, wavefront wv from line wv (64 / LR) on, a lane the points
+    // li and LR + li of the line's span; up to four lines' loads in flight before
+    // their LDS stores
     {
         const int nlines = 9 * nfull;
-        int xa = x0 - 1 + lane, xb = x0 + 63 + lane;
+        constexpr int LW = 64 / LR, LSTEP = 4 * LW;   // lines per wavefront, workgroup
+        const int li = lane % LR;
+        int xa = x0 - 1 + li, xb = x0 + LR - 1 + li;
         xa = xa < 0 ? xa + NXAA : xa;
         xb = xb >= NXAA ? xb - NXAA : xb;
-        const bool hasb = lane < span - 64;
-        for (int L0 = wv; L0 < nlines; L0 += 16) {
+        const bool hasb = li < span - LR;
+        for (int L0 = wv * LW + lane / LR; L0 < nlines; L0 += 4 * LSTEP) {
             double va[4], vb[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int L = L0 + 4 * i;
+                const int L = L0 + LSTEP * i;
                 if (L < nlines) {
                     const int o = L / nfull, f = L - o * nfull;
                     const int dz = o / 3 - 1, dy = o - 3 * (o / 3) - 1;
@@ -1269,10 +1278,10 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int L = L0 + 4 * i;
+                const int L = L0 + LSTEP * i;
                 if (L < nlines) {
-                    tile[L * span + lane] = va[i];
-                    if (hasb) tile[L * span + 64 + lane] = vb[i];
+                    tile[L * span + li] = va[i];
+                    if (hasb) tile[L * span + LR + li] = vb[i];
                 }
             }
         }
@@ -1316,23 +1325,23 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
         if (32 * k < kp) {
-            const cbf8 a = *reinterpret_cast<const cbf8 *>(&As[(16 * wv + fr) * ldk + 32 * k + fk]);
+            const cbf8 a = *reinterpret_cast<const cbf8 *>(&As[(wr + fr) * ldk + 32 * k + fk]);
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bfr[k][j], acc[j], 0, 0, 0);
         }
     }
     // epilogue through LDS (the operand tiles are done with): the tile's H
-    // rows, their BF16 copy and its two 32-row blocks of the tiled transposed
+    // rows, their BF16 copy and its 32-row blocks of the tiled transposed
     // layout are each one contiguous run of memory, written with 16-byte stores
     __syncthreads();
     constexpr int LDH = W + 4;
     float *Hs = reinterpret_cast<float *>(As);   // [LR][LDH]
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const int gn = 16 * j + fr;
+        const int gn = wc + 16 * j + fr;
         const float bias = b0[gn];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) Hs[(16 * wv + rq + q) * LDH + gn] = acc[j][q] + bias;
+        for (int q = 0; q < 4; ++q) Hs[(wr + rq + q) * LDH + gn] = acc[j][q] + bias;
     }
     __syncthreads();
     float4 *Ho = reinterpret_cast<float4 *>(H + r0 * W);
@@ -1368,7 +1377,15 @@ __global__ __launch_bounds__(256) void k_closure_lift(const double *__restrict__
     }
 }
 
-// tau[q][z][y][x] = (H16 Wp + bp) std + mean for LIFT_ROWS rows of the chunk:
+using LiftKernel = void (*)(const double *, const double *, int, int, int, int, int, int, int, int, const float *,
+                            const float *, const unsigned short *, const float *, float *, unsigned short *,
+                            unsigned short *);
+LiftKernel lift_kernel(int width, int rows) {
+    if (rows == 64) return width == 32 ? k_closure_lift<32, 64> : k_closure_lift<64, 64>;
+    return width == 32 ? k_closure_lift<32, 32> : k_closure_lift<64, 32>;
+}
+
+// tau[q][z][y][x] = (H16 Wp + bp) std + mean for PROJ_ROWS rows of the chunk:
 // the network's projection on MFMA with the K order and epilogue of nn::gemm
 // and nn::bias_act, the unpacking of k_closure_unpack, in one pass (the
 // outputs of a tile are staged in LDS so that each variable's 64 values are
@@ -1379,7 +1396,7 @@ __global__ __launch_bounds__(256) void k_closure_project(const unsigned short *_
                                                          const float *__restrict__ bp, int cout, int z0, int N2,
                                                          int NZAA, const float *__restrict__ mu,
                                                          const float *__restrict__ sd, double *__restrict__ tau) {
-    constexpr int LR = LIFT_ROWS, LDB = W + 8, KS = W / 32;
+    constexpr int LR = PROJ_ROWS, LDB = W + 8, KS = W / 32;
     __shared__ __align__(16) unsigned short Bs[16 * LDB];
     __shared__ double outs[16 * LR];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, fr = lane & 15, fk = 8 * (lane >> 4);
@@ -1449,19 +1466,14 @@ void closure_correction(coral_amd_ctx &c) {
             const int np = std::min(cl.chunk, P.NZAA - z0);
             const unsigned g = unsigned(((long long)np * N2 + 255) / 256);
             if (cl.fused_io) {
-                const LiftShape ls = lift_shape(P.nfull, cl.net.cin, cl.net.width);
-                const unsigned nt = unsigned((long long)np * N2 / LIFT_ROWS);
+                const int rows = lift_rows(P.NXAA);
+                const LiftShape ls = lift_shape(P.nfull, cl.net.cin, cl.net.width, rows);
+                const unsigned nt = unsigned((long long)np * N2 / PROJ_ROWS);
                 unsigned short *h16t = nn::net_tiled(cl.net, cl.ws) ? cl.ws.H16T : nullptr;
-                const unsigned short *W0 = cl.W0T.p;
-                const float *b0 = cl.net.w + cl.net.off_b0;
-                if (cl.net.width == 32)
-                    hipLaunchKernelGGL(k_closure_lift<32>, dim3(nt), dim3(256), ls.bytes, c.stream, cl.phys_full.p,
-                                       cl.zgrid.p, z0, P.NXAA, P.NYAA, P.NZAA, P.nfull, cl.net.cin, ls.kp, ls.ldk,
-                                       cl.mu_in.p, cl.sd_in.p, W0, b0, cl.ws.H, cl.ws.H16, h16t);
-                else
-                    hipLaunchKernelGGL(k_closure_lift<64>, dim3(nt), dim3(256), ls.bytes, c.stream, cl.phys_full.p,
-                                       cl.zgrid.p, z0, P.NXAA, P.NYAA, P.NZAA, P.nfull, cl.net.cin, ls.kp, ls.ldk,
-                                       cl.mu_in.p, cl.sd_in.p, W0, b0, cl.ws.H, cl.ws.H16, h16t);
+                hipLaunchKernelGGL(lift_kernel(cl.net.width, rows), dim3(unsigned((long long)np * N2 / rows)), dim3(256),
+                                   ls.bytes, c.stream, cl.phys_full.p, cl.zgrid.p, z0, P.NXAA, P.NYAA, P.NZAA, P.nfull,
+                                   cl.net.cin, ls.kp, ls.ldk, cl.mu_in.p, cl.sd_in.p, cl.W0T.p,
+                                   cl.net.w + cl.net.off_b0, cl.ws.H, cl.ws.H16, h16t);
                 check_launch("closure lift");
                 nn::net_forward(c.stream, cl.net, nullptr, np, nullptr, cl.ws);
                 const unsigned short *Wp = cl.net.w16 + cl.net.off_Wp;
@@ -2941,22 +2953,18 @@ int coral_amd_set_closure(coral_amd_ctx *c, const coral_amd_closure *cl) {
             C.ws.mwork = C.mwork.p;
             C.ws.nmwork = nn::modes_work(nbp, N2, n.width, C.chunk);
         }
-        // the fused lift / projection: tiles inside x-lines, at most 16 outputs,
+        // the fused lift / projection: tiles inside x-lines and planes, at most 16 outputs,
         // their dynamic LDS within the device limit (CORAL_AMD_CLOSURE_UNFUSED=1
         // keeps the pack, GEMM and unpack kernels)
         {
             const char *ev = std::getenv("CORAL_AMD_CLOSURE_UNFUSED");
-            const LiftShape ls = lift_shape(P.nfull, n.cin, n.width);
-            C.fused_io = !(ev && ev[0] == '1') && P.NXAA % LIFT_ROWS == 0 && n.cout <= 16 &&
+            const int rows = lift_rows(P.NXAA);
+            const LiftShape ls = lift_shape(P.nfull, n.cin, n.width, std::max(rows, 32));
+            C.fused_io = !(ev && ev[0] == '1') && rows > 0 && N2 % PROJ_ROWS == 0 && n.cout <= 16 &&
                          (n.width == 32 || n.width == 64) && ls.kp <= 256 && ls.bytes <= 65536;
-            if (C.fused_io && ls.bytes > 49152) {
-                if (n.width == 32)
-                    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_closure_lift<32>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(ls.bytes)));
-                else
-                    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_closure_lift<64>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(ls.bytes)));
-            }
+            if (C.fused_io && ls.bytes > 49152)
+                HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(lift_kernel(n.width, rows)),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(ls.bytes)));
             if (C.fused_io) {   // no packed input rows or FP32 outputs to keep
                 C.X16.alloc(0);
                 C.Y.alloc(0);
