@@ -84,6 +84,7 @@ EXPORTS = (
     "coral_amd_set_source", "coral_amd_set_fixed_physical", "coral_amd_set_smagorinsky", "coral_amd_nn_mode_scale_t", "coral_amd_nn_modes_supported",
     "coral_amd_nn_modes_work", "coral_amd_nn_modes", "coral_amd_nn_tile_transpose",
     "coral_amd_nn_gemm_bias", "coral_amd_nn_gemm16", "coral_amd_nn_gemm_gelu_bwd",
+    "coral_amd_nn_gemm_gelu_bwd_work",
 )
 
 
