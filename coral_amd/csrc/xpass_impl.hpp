@@ -234,8 +234,33 @@ struct PairMax {
 };
 template <class T>
 __device__ inline T bal_scale(unsigned mbits) { return bal_pow<T>(mbits, -1); }
+// A line with an infinity or a NaN stays by itself, as where every line has a
+// sequence of its own: the packing leaves its values out of the pair (a branch
+// that is not taken otherwise; the empty asm keeps it from being turned into a
+// select per value), and the scaling back makes every value of the line a NaN.
+// Costs 1 % of the pass: us per launch 753 -> 759 at 288^2 x 97, 233 -> 236 at
+// 192^2 x 65, 26.5 -> 27.0 at 72 x 48 x 41.
 template <class T>
-__device__ inline T bal_unscale(unsigned mbits) { return bal_pow<T>(mbits, +1); }
+__device__ inline bool bal_bad(unsigned mbits) {
+    return mbits >= (sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u);
+}
+template <class T>
+__device__ inline T bal_unscale(unsigned mbits) {
+    return bal_bad<T>(mbits) ? T(__builtin_nanf("")) : bal_pow<T>(mbits, +1);
+}
+template <class V, int K>
+__device__ inline void leave_out(bool bad, V (&v)[K]) {
+    if (bad) {
+        asm volatile("");
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            if constexpr (std::is_floating_point<V>::value)
+                v[r] = 0;
+            else
+                v[r] = mkc<V>(0, 0);
+        }
+    }
+}
 
 // forward transforms of product pair pq (products 2 pq, 2 pq + 1) of the
 // group's lines and the store of the kept kx
@@ -285,6 +310,8 @@ __device__ inline void xfwd_pair(const XPassArgs &a, const C (&fv)[XShape<P>::NT
             const int t = lane + LN * c, l = t / TL, j = t - l * TL;
             if (!X::FULL && t >= LPW * TL) break;
             const T s0 = bal_scale<T>(pm.first(l)), s1 = bal_scale<T>(pm.second(l));
+            leave_out(bal_bad<T>(pm.first(l)), p0[c]);
+            leave_out(bal_bad<T>(pm.second(l)), p1[c]);
             C y[RL];
 #pragma unroll
             for (int r = 0; r < RL; ++r) y[r] = mkc<C>(p0[c][r] * s0, p1[c][r] * s1);
@@ -430,6 +457,8 @@ __global__ __launch_bounds__(256) void k_xpass_wave(XPassArgs a, const C *__rest
                 if (TOT % LN == 0 || b < TOT) {
                     const int l = b / T0, j = b - l * T0;
                     const T sa = bal_scale<T>(pm.first(l)), sb = bal_scale<T>(pm.second(l));
+                    leave_out(bal_bad<T>(pm.first(l)), va[c]);
+                    leave_out(bal_bad<T>(pm.second(l)), vb[c]);
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
                         const int e = j + r * T0;
@@ -464,8 +493,14 @@ __global__ __launch_bounds__(256) void k_xpass_wave(XPassArgs a, const C *__rest
                     const C *g1 = G + ((size_t)(has1 ? f1 : f0) * nlines + lo) * NK;
                     T sa = 1, sb = 1;
                     if constexpr (x_balanced<N, C>()) {
-                        sa = bal_scale<T>(pm.first(l));
-                        sb = bal_scale<T>(pm.second(l));
+                        // a line left out: its partner's values in its place
+                        const bool bad0 = bal_bad<T>(pm.first(l)), bad1 = bal_bad<T>(pm.second(l));
+                        const unsigned ma = bad0 ? pm.second(l) : pm.first(l), mb = bad1 ? pm.first(l) : pm.second(l);
+                        const C *h0 = g0;
+                        g0 = bad0 ? g1 : g0;
+                        g1 = bad1 ? h0 : g1;
+                        sa = bal_scale<T>(ma);
+                        sb = bal_scale<T>(mb);
                     }
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
