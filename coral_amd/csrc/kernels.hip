@@ -2110,8 +2110,8 @@ __global__ __launch_bounds__(64) void k_solve16_batch(const Solve16Args *__restr
 bool solve16_shape(const Solve16Args &a, Solve16Shape &sh) {
     if (a.kl > 16 || a.n < 1 || a.ncol16 < 16 * ((a.n + 15) / 16 + 1) || !a.ucol || !a.sink) return false;
     if (a.nslot < 1 || a.nslot > SOLVE16_SLOTS || (a.nslot > 1 && !a.mem)) return false;
-    sh.nq = 1 + (a.kv + 15) / 16;
-    if (sh.nq < 2 || sh.nq > 4) return false;
+    sh.nq = std::max(2, 1 + (a.kv + 15) / 16);   // (a diagonal system: the second register takes zeros)
+    if (sh.nq > 4) return false;
     // Two right-hand sides per wavefront read the factors once for both and
     // share the step's masks and addresses, but take 1.35 times one's chain of
     // steps: below a wavefront per SIMD (1024) that chain is the launch time.
@@ -2242,7 +2242,7 @@ void solve16_trim_u_copy(hipStream_t st, const void *Ufull, int elem, int n, int
 
 int solve16_ncol(int n, int kl, int kv) {
     // (positions are packed in 14 bits of the position words)
-    if (kl > 16 || n < 1 || (n < 32 && kv < 1) || n >= SOLVE16_NONE || 1 + (kv + 15) / 16 > 4) return 0;
+    if (kl > 16 || n < 1 || n >= SOLVE16_NONE || 1 + (kv + 15) / 16 > 4) return 0;
     return 16 * ((n + 15) / 16 + 1);
 }
 

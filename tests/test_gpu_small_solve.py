@@ -23,7 +23,7 @@ def solver_mod():
 
 
 @pytest.mark.parametrize("n", [1, 2, 5, 15, 16, 17, 31, 32, 33])
-@pytest.mark.parametrize("kl,ku", [(0, 1), (1, 0), (1, 2), (5, 4), (15, 16), (16, 27)])
+@pytest.mark.parametrize("kl,ku", [(0, 0), (0, 1), (1, 0), (1, 2), (5, 4), (15, 16), (16, 27)])
 def test_short_systems(solver_mod, n, kl, ku):
     rng = np.random.default_rng(100 * n + kl)
     ns = 6   # a full wavefront of four systems and a part of one
