@@ -50,6 +50,7 @@ class HostCopy {
     template <class Dst, class Fill>
     void to_host(hipStream_t st, const void *dev, size_t nrow, size_t row_bytes, Dst dst, Fill fill) {
         if (nrow == 0 || row_bytes == 0) return fill(0, 1);
+        std::lock_guard<std::mutex> one(use_);
         const Plan p = plan(nrow, row_bytes);
         Task task(*this, p.nchunk, 0, fill, [&](size_t c) {
             const char *s = slot(p, c);
@@ -73,6 +74,7 @@ class HostCopy {
     template <class Src>
     void to_device(hipStream_t st, void *dev, size_t nrow, size_t row_bytes, Src src) {
         if (nrow == 0 || row_bytes == 0) return;
+        std::lock_guard<std::mutex> one(use_);
         const Plan p = plan(nrow, row_bytes);
         Task task(*this, p.nchunk, p.nslot, nullptr, [&](size_t c) {
             char *s = slot(p, c);
@@ -213,6 +215,7 @@ class HostCopy {
         }
     }
 
+    std::mutex use_;   // one copy at a time: callers on several threads share the slots
     char *slab_ = nullptr;
     size_t bytes_ = 0;
     std::vector<hipEvent_t> ev_;

@@ -36,3 +36,20 @@ def test_states_and_volumes_round_trip(native_lib, grid):
         assert np.linalg.norm(c - a) <= 1e-12 * np.linalg.norm(a)
         g.set_variable_physical("kxky", 0, 3, v)      # the tables of its first use again
         assert np.array_equal(g.get_field("kxky", 0), c)
+
+
+def test_two_threads_read_one_run(native_lib):
+    """Threads that read states of one run at the same time (the calls release
+    the interpreter's lock) each get the whole state."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from coral_amd import solver
+    r = product_recipe("coral.equations.rbc_ra1e5")
+    rng = np.random.default_rng(4)
+    with solver.Solver(r, 64, 96, 65, 2.0, 3.0) as g:
+        shape = (32, 144, g.totals[0])
+        g.set_field("kxky", 0, rng.standard_normal(shape) + 1j * rng.standard_normal(shape))
+        want = g.get_field("kxky", 0)
+        with ThreadPoolExecutor(4) as ex:
+            for got in ex.map(lambda _: g.get_field("kxky", 0), range(16)):
+                assert np.array_equal(got, want)
