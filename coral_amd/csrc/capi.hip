@@ -137,9 +137,8 @@ struct TimerRec {
 }  // namespace
 
 struct coral_amd_ctx {
-    // host copies: pinned chunks, and a device array in the host's layout
+    // host copies through pinned chunks
     HostCopy host;
-    DevBuf<double2> hostd;
     // stencil tables of coupled variables (coral_amd_get/set_variable_physical),
     // built at a variable's first use
     std::map<std::pair<int, int>, std::unique_ptr<VarDev>> var_dev;
@@ -1794,15 +1793,31 @@ void transpose(hipStream_t st, const TI *in, int R, int C, size_t ir, size_t ib,
 
 // Host layouts are formed on the device and copied as they are: a volume's
 // transposition on one host core took longer than everything else about it.
-void ensure_hostd(coral_amd_ctx &c, size_t n) {
-    if (c.hostd.n < n) c.hostd.alloc(n);
-}
+// n values in the host's layout: room in the x spectra of the products or of the
+// full variables, which hold nothing between two calls (and nothing that a copy
+// out is formed from: it is formed from Qhat or physd).  They are large enough
+// but for recipes with at most one variable of each kind, where the array is
+// freed with this object.
+struct HostLayout {
+    double2 *p;
+    DevBuf<double2> own;
+    HostLayout(coral_amd_ctx &c, size_t n) {
+        if (c.H.n >= n) {
+            p = c.H.p;
+        } else if (c.G.n >= n) {
+            p = c.G.p;
+        } else {
+            own.alloc(n);
+            p = own.p;
+        }
+    }
+};
 
 // device [z][y][x] -> host [x][y][z]
 void download_phys(coral_amd_ctx &c, double *out) {
     const Problem &P = c.P;
-    ensure_hostd(c, (c.physd.n + 1) / 2);
-    double *d = reinterpret_cast<double *>(c.hostd.p);
+    const HostLayout h(c, (c.physd.n + 1) / 2);
+    double *d = reinterpret_cast<double *>(h.p);
     const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
     transpose(c.stream, c.physd.p, P.NZAA, P.NXAA, NY * NX, NX, d, NY * NZ, NZ, P.NYAA);
     c.host.to_host(c.stream, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return out + x * NY * NZ; },
@@ -1813,8 +1828,8 @@ void download_phys(coral_amd_ctx &c, double *out) {
 void upload_phys(coral_amd_ctx &c, const double *in) {
     const Problem &P = c.P;
     ensure_phys(c);
-    ensure_hostd(c, (c.physd.n + 1) / 2);
-    double *d = reinterpret_cast<double *>(c.hostd.p);
+    const HostLayout h(c, (c.physd.n + 1) / 2);
+    double *d = reinterpret_cast<double *>(h.p);
     const size_t NX = P.NXAA, NY = P.NYAA, NZ = P.NZAA;
     c.host.to_device(c.stream, d, NX, NY * NZ * sizeof(double), [&](size_t x) { return in + x * NY * NZ; });
     transpose(c.stream, d, P.NXAA, P.NZAA, NY * NZ, NZ, c.physd.p, NY * NX, NX, P.NYAA);
@@ -2495,12 +2510,12 @@ int coral_amd_products(coral_amd_ctx *c, double *out) {
         join_mean(*c);
         // [q][n][s] -> [q][s][n] on the device, then [q][ix][y slot][n]
         const size_t nsys = P.nsys, per = nsys * P.NZ;
-        ensure_hostd(*c, per * P.nquad);
+        const HostLayout h(*c, per * P.nquad);
         if (fp32)
-            transpose(c->stream, c->Qhat32.p, P.NZ, P.nsys, nsys, per, c->hostd.p, P.NZ, per, P.nquad);
+            transpose(c->stream, c->Qhat32.p, P.NZ, P.nsys, nsys, per, h.p, P.NZ, per, P.nquad);
         else
-            transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, nsys, per, c->hostd.p, P.NZ, per, P.nquad);
-        download_modes(*c, c->hostd.p, P.nquad, P.NZ, out);
+            transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, nsys, per, h.p, P.NZ, per, P.nquad);
+        download_modes(*c, h.p, P.nquad, P.NZ, out);
         return 0;
     } catch (const std::exception &e) {
         return fail(e);
@@ -2513,9 +2528,9 @@ int coral_amd_bwd_transform(coral_amd_ctx *c, const double *spec, double *phys) 
         const Problem &P = c->P;
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        ensure_hostd(*c, size_t(P.nsys) * P.NZ);
-        upload_modes(*c, spec, P.NZ, c->hostd.p);
-        transpose(c->stream, c->hostd.p, P.nsys, P.NZ, P.NZ, 0, c->spec.p, P.nsys, 0, 1);
+        const HostLayout h(*c, size_t(P.nsys) * P.NZ);
+        upload_modes(*c, spec, P.NZ, h.p);
+        transpose(c->stream, h.p, P.nsys, P.NZ, P.NZ, 0, c->spec.p, P.nsys, 0, 1);
         zbwd(*c, c->spec.p, c->Fz.p, 1);
         launch_ybwd(c->stream, c->py, c->Fz.p, c->G.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
         const long long nlines = (long long)P.NZAA * P.NYAA;
@@ -2540,9 +2555,9 @@ int coral_amd_fwd_transform(coral_amd_ctx *c, const double *phys, double *spec) 
         launch_yfwd(c->stream, c->py, c->H.p, c->Hy.p, 1, P.NZAA, P.nkx, P.nky, P.NY);
         zfwd(*c, c->Hy.p, c->Qhat.p, 1);
         HIP_OK(hipStreamSynchronize(c->stream));
-        ensure_hostd(*c, size_t(P.nsys) * P.NZ);
-        transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, P.nsys, 0, c->hostd.p, P.NZ, 0, 1);
-        download_modes(*c, c->hostd.p, 1, P.NZ, spec);
+        const HostLayout h(*c, size_t(P.nsys) * P.NZ);
+        transpose(c->stream, c->Qhat.p, P.NZ, P.nsys, P.nsys, 0, h.p, P.NZ, 0, 1);
+        download_modes(*c, h.p, 1, P.NZ, spec);
         return 0;
     } catch (const std::exception &e) {
         return fail(e);

@@ -53,3 +53,36 @@ def test_two_threads_read_one_run(native_lib):
         with ThreadPoolExecutor(4) as ex:
             for got in ex.map(lambda _: g.get_field("kxky", 0), range(16)):
                 assert np.array_equal(got, want)
+
+
+def _free_bytes():
+    import ctypes
+
+    from coral_amd import devmem
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert devmem.hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_reading_keeps_no_device_memory(native_lib):
+    """Products, fields, variables and transforms leave only the volume that the
+    physical fields are formed in and the small tables of a variable."""
+    from coral_amd import solver
+    r = product_recipe("coral.equations.rbc_ra1e5")
+    rng = np.random.default_rng(5)
+    with solver.Solver(r, 96, 96, 65, 2.0, 2.0) as g:
+        shape = (48, 144, g.totals[0])
+        g.set_field("kxky", 0, rng.standard_normal(shape) + 1j * rng.standard_normal(shape))
+        g.factorize_operators(1e-5)
+        g.march_forward(1e-5, 1)
+        volume = 8 * 144 * 144 * 97
+        start = _free_bytes()
+        g.physical(0)
+        q = g.products()
+        g.bwd_transform(q[0])
+        v = g.variable_physical("kxky", 0, 2)
+        g.fwd_transform(v)
+        g.set_variable_physical("kxky", 0, 2, v)
+        # the allocator hands out memory in pieces of up to 4 MiB; the spectra of
+        # the nine products in the host's layout are 42 MB
+        assert start - _free_bytes() <= volume + (8 << 20)
