@@ -3372,9 +3372,21 @@ void ens_capture(coral_amd_ensemble &e) {
     e.epar = 0;
 }
 
-// whether the runs can step in lockstep: the same number of stages and no
-// residual refinement (the batched solves leave it out)
+// whether the runs can step in lockstep: the same number of stages, no
+// residual refinement (the batched solves leave it out), and a HIP runtime from
+// 7.2 on.  With the 7.0 runtime that a PyTorch build brings into the process, the
+// capture ended the process in a segmentation fault of the host; nothing in this
+// file explains it, and on 7.2 the same calls are tested bit for bit.
+constexpr int LOCKSTEP_RUNTIME = 70200000;
 bool ens_lockstep_ok(const coral_amd_ensemble &e, std::string *why = nullptr) {
+    int v = 0;
+    HIP_OK(hipRuntimeGetVersion(&v));
+    if (v < LOCKSTEP_RUNTIME) {
+        if (why)
+            *why = "lockstep steps need HIP runtime 7.2 or later, this process has " + std::to_string(v / 10000000) +
+                   "." + std::to_string(v / 100000 % 100);
+        return false;
+    }
     for (auto *c : e.runs) {
         if (c->P.nstages != e.runs[0]->P.nstages) {
             if (why) *why = "lockstep steps need the same IMEX scheme on every run";

@@ -405,8 +405,9 @@ int coral_amd_ensemble_destroy(coral_amd_ensemble *ens);
  * which, stage by stage, every run's NL terms and right-hand sides (spread
  * over max(1, -nbranch) parallel branches) are followed by the stage's kxky
  * solves of all runs as one batched launch per kernel variant (same results
- * bit for bit); it needs the same IMEX scheme on every run and no residual
- * refinement. */
+ * bit for bit); it needs the same IMEX scheme on every run, no residual
+ * refinement and HIP runtime 7.2 or later (refused otherwise; the tuner then
+ * leaves it out). */
 int coral_amd_ensemble_set_schedule(coral_amd_ensemble *ens, int32_t nbranch, const int32_t *assign);
 /* The tuner: for every run, each launch shape (x pass 4, 2 or 1 wavefronts per
  * workgroup; z transforms on MFMA or as vector GEMMs) timed over trial_steps

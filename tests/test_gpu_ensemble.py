@@ -137,3 +137,42 @@ def test_lockstep_ensemble_matches_solo_runs(mods):
     r0.close()
     for g, _ in runs:
         g.close()
+
+
+def test_lockstep_is_refused_under_an_older_runtime(native_lib):
+    """With PyTorch's own HIP runtime (before 7.2) in the process the lockstep
+    schedule is an error, and the schedules of branches are still set."""
+    import os
+    import subprocess
+    import sys
+
+    from conftest import ROOT
+    code = """
+import ctypes, glob, os
+import numpy as np
+import torch
+so = glob.glob(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so*"))
+v = ctypes.c_int()
+assert not so or ctypes.CDLL(so[0]).hipRuntimeGetVersion(ctypes.byref(v)) == 0
+if not so or v.value >= 70200000:
+    print("SKIP", v.value)
+    raise SystemExit
+from coral_amd import ensemble, solver
+r = ensemble.rbc_recipe(1e5, 1.0)
+runs = [solver.Solver(r, 16, 16, 17, 2.0, 2.0) for _ in range(2)]
+with ensemble.Ensemble(runs) as ens:
+    for nb in (0, -2):
+        try:
+            ens.set_schedule(nb)
+        except Exception as e:
+            assert "HIP runtime 7.2" in str(e), e
+        else:
+            raise AssertionError("lockstep accepted")
+    ens.set_schedule(2)
+print("REFUSED")
+"""
+    p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                       text=True, timeout=100)
+    if "SKIP" in p.stdout:
+        pytest.skip("PyTorch's HIP runtime is not older")
+    assert p.returncode == 0 and "REFUSED" in p.stdout, p.stdout
