@@ -10,10 +10,12 @@
 //   NL insertion            PL_IMEX_timestepping_marching.f90:306-350
 #include "assembly.hpp"
 
-#include <functional>
-#include <array>
 #include <algorithm>
+#include <array>
 #include <cmath>
+#include <cstdint>
+#include <cstring>
+#include <functional>
 #include <map>
 #include <stdexcept>
 
@@ -242,21 +244,56 @@ static void find_real_form(const coral_amd_system &s, SystemTables &t) {
 // (i kx)^a (i ky)^b becomes (-1)^b times itself (reflection), or (-1)^b
 // (i kx)^b (i ky)^a (rotation).  The search runs over the involutions of the
 // variables (swapping only variables of one boundary-condition code) and of
-// the equations (of one order); for each, the signs are a two-colouring of the
-// graph (equation, variable) whose edges are the pieces, which must map onto
-// pieces of equal magnitude.
+// the equations (of one order) that exchange equal pieces up to signs, as far as
+// one variable or equation shows; for each pair, the signs are a two-colouring of
+// the graph (equation, variable) whose edges are the pieces, which must map onto
+// pieces of equal magnitude.  The recipes of this repository leave one pair to
+// look at; systems of many alike equations could leave 764 squared at eight
+// variables (seconds), so the search gives up after MAX_PAIRS (milliseconds) and
+// every wavenumber is then factored.
 static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotate, SystemTables::Symmetry &sym) {
+    constexpr int MAXV = 8, MAX_PAIRS = 2000;
     const int nv = s.nvars;
-    if (nv > 8) return;   // 764 involutions each at 8
-    // coefficients by (mass or stiffness, equation, variable, iz, mz, a, b)
-    std::map<std::array<int, 7>, double> c;
+    if (nv > MAXV) return;
+    // coefficients by (mass or stiffness, equation, variable, iz, mz, a, b), sorted
+    typedef std::array<int, 7> Key;
+    std::vector<std::pair<Key, double>> c;
+    c.reserve(s.n_mass + s.n_stif);
     for (int k = 0; k < s.n_mass + s.n_stif; ++k) {
         const coral_amd_piece &p = k < s.n_mass ? s.mass[k] : s.stif[k - s.n_mass];
-        if (p.dsca != 0.0) c[{k < s.n_mass ? 0 : 1, p.eqn, p.var, p.iz, p.mz, p.kx, p.ky}] += p.dsca;
+        if (!std::isfinite(p.dsca)) return;
+        if (p.dsca != 0.0) c.push_back({{k < s.n_mass ? 0 : 1, p.eqn, p.var, p.iz, p.mz, p.kx, p.ky}, p.dsca});
     }
-    auto involutions = [nv](const int32_t *kind) {
-        std::vector<std::vector<int>> out;
-        std::vector<int> cur(nv, -1);
+    const auto by_key = [](const auto &x, const auto &y) { return x.first < y.first; };
+    std::stable_sort(c.begin(), c.end(), by_key);
+    size_t n = 0;   // pieces of one key are added in their order
+    for (size_t k = 0; k < c.size(); ++k) {
+        if (n > 0 && c[n - 1].first == c[k].first)
+            c[n - 1].second += c[k].second;
+        else
+            c[n++] = c[k];
+    }
+    c.resize(n);
+    // involutions of the variables or equations: i and j may be exchanged where
+    // their kinds are equal and the pieces of i, mapped, look like those of j (by
+    // sums of hashes; whether they are is checked below)
+    auto involutions = [&](const int32_t *kind, int which) {
+        std::array<uint64_t, MAXV> at{}, mapped{};
+        for (const auto &[k, val] : c) {
+            const double mag = std::fabs(val);
+            uint64_t h;
+            std::memcpy(&h, &mag, sizeof h);
+            const auto mix = [](uint64_t x, uint64_t y) {
+                x = (x ^ y) * 0x9E3779B97F4A7C15ull;
+                return x ^ (x >> 29);
+            };
+            h = mix(mix(mix(h, k[0] + 1), k[3] + 1), k[4] + 1);
+            at[k[which]] += mix(mix(h, k[5] + 1), k[6] + 1);
+            mapped[k[which]] += rotate ? mix(mix(h, k[6] + 1), k[5] + 1) : mix(mix(h, k[5] + 1), k[6] + 1);
+        }
+        std::vector<std::array<int, MAXV>> out;
+        std::array<int, MAXV> cur;
+        cur.fill(-1);
         std::function<void(int)> go = [&](int i) {
             while (i < nv && cur[i] >= 0) ++i;
             if (i == nv) {
@@ -264,7 +301,7 @@ static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotat
                 return;
             }
             for (int j = i; j < nv; ++j) {
-                if (cur[j] >= 0 || kind[i] != kind[j]) continue;
+                if (cur[j] >= 0 || kind[i] != kind[j] || mapped[i] != at[j] || mapped[j] != at[i]) continue;
                 cur[i] = j;
                 cur[j] = i;
                 go(i + 1);
@@ -274,41 +311,39 @@ static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotat
         go(0);
         return out;
     };
-    const auto vars = involutions(s.bc_codes), eqns = involutions(s.eqn_orders);
+    const auto vars = involutions(s.bc_codes, 2), eqns = involutions(s.eqn_orders, 1);
+    int tried = 0;
     for (const auto &pe : eqns)
         for (const auto &pv : vars) {
-            // edges (equation of k', variable of k', parity of the sign), checked for magnitude
+            if (++tried > MAX_PAIRS) return;
+            // signs relative to a root, joined piece by piece: rel[x] is the sign of
+            // equation x (or variable x - nv) against that of up[x]
+            std::array<int, 2 * MAXV> up;
+            std::array<unsigned char, 2 * MAXV> rel{};
+            for (int x = 0; x < 2 * nv; ++x) up[x] = x;
+            auto root = [&](int x, unsigned char &neg) {
+                neg = 0;
+                for (; up[x] != x; x = up[x]) neg ^= rel[x];
+                return x;
+            };
             bool ok = true;
-            std::vector<std::vector<std::pair<int, int>>> adj(2 * nv);
             for (const auto &[key, val] : c) {
                 const auto [op, e, v, iz, mz, a, b] = key;   // at k' : (e, v)
-                const auto it = c.find({op, pe[e], pv[v], iz, mz, rotate ? b : a, rotate ? a : b});
-                if (it == c.end() || std::fabs(it->second) != std::fabs(val)) {
+                const Key to{op, pe[e], pv[v], iz, mz, rotate ? b : a, rotate ? a : b};
+                const auto it = std::lower_bound(c.begin(), c.end(), std::make_pair(to, 0.0), by_key);
+                if (it == c.end() || it->first != to || !(std::fabs(it->second) == std::fabs(val))) {
                     ok = false;
                     break;
                 }
-                const int par = ((b & 1) != 0) ^ ((it->second < 0) != (val < 0));
-                adj[e].push_back({nv + v, par});
-                adj[nv + v].push_back({e, par});
-            }
-            if (!ok) continue;
-            std::vector<int> neg(2 * nv, -1);
-            for (int root = 0; root < 2 * nv && ok; ++root) {
-                if (neg[root] >= 0) continue;
-                neg[root] = 0;
-                std::vector<int> stack{root};
-                while (!stack.empty() && ok) {
-                    const int u = stack.back();
-                    stack.pop_back();
-                    for (auto [w, par] : adj[u]) {
-                        if (neg[w] < 0) {
-                            neg[w] = neg[u] ^ par;
-                            stack.push_back(w);
-                        } else if (neg[w] != (neg[u] ^ par)) {
-                            ok = false;
-                            break;
-                        }
-                    }
+                const unsigned char par = ((b & 1) != 0) ^ ((it->second < 0) != (val < 0));
+                unsigned char ne, nw;
+                const int re = root(e, ne), rw = root(nv + v, nw);
+                if (re != rw) {
+                    up[re] = rw;
+                    rel[re] = ne ^ nw ^ par;
+                } else if ((ne ^ nw) != par) {
+                    ok = false;
+                    break;
                 }
             }
             if (!ok) continue;
@@ -319,15 +354,18 @@ static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotat
             sym.cneg.assign(t.total, 0);
             for (int i = 0; i < nv; ++i) {
                 // (pe and pv are their own inverses)
+                unsigned char ne, nw;
+                root(pe[i], ne);
+                root(nv + pv[i], nw);
                 for (int r = 0; r < t.eqn_size[i]; ++r) {
                     const int at = t.posQ[t.eqn_first[i] + r];
                     sym.row[at] = t.posQ[t.eqn_first[pe[i]] + r];
-                    sym.rneg[at] = (unsigned char)neg[pe[i]];
+                    sym.rneg[at] = ne;
                 }
                 for (int r = 0; r < t.var_size[i]; ++r) {
                     const int at = t.posP[t.var_first[i] + r];
                     sym.col[at] = t.posP[t.var_first[pv[i]] + r];
-                    sym.cneg[at] = (unsigned char)neg[nv + pv[i]];
+                    sym.cneg[at] = nw;
                 }
             }
             return;
