@@ -14,6 +14,7 @@
 #include <array>
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
@@ -370,6 +371,55 @@ static void find_symmetry(const coral_amd_system &s, SystemTables &t, bool rotat
             }
             return;
         }
+}
+
+FactorSharing factor_sharing(const SystemTables &t, int nkx, int NY, bool square_box) {
+    FactorSharing f;
+    const bool refl = t.reflect.found, rota = t.rotate.found && square_box;
+    if (!refl && !rota) return f;
+    // the partners of (kx, ky), in the order of f.sym
+    auto partners = [&](int kx, int ky) {
+        std::vector<std::pair<int, int>> out;
+        if (refl) out.push_back({kx, -ky});
+        if (rota) out.push_back({ky, -kx});
+        if (refl && rota) out.push_back({ky, kx});
+        return out;
+    };
+    if (refl) f.sym.push_back(t.reflect);
+    if (rota) f.sym.push_back(t.rotate);
+    if (refl && rota) {   // the reflection after the rotation
+        SystemTables::Symmetry c = t.rotate;
+        for (int i = 0; i < t.total; ++i) {
+            c.rneg[i] ^= t.reflect.rneg[c.row[i]];
+            c.cneg[i] ^= t.reflect.cneg[c.col[i]];
+            c.row[i] = t.reflect.row[c.row[i]];
+            c.col[i] = t.reflect.col[c.col[i]];
+        }
+        f.sym.push_back(c);
+    }
+    f.nslot = 1 + int(f.sym.size());
+    const int nky = NY - 1;
+    auto index = [&](int kx, int ky) {
+        if (kx < 0 || kx >= nkx || std::abs(ky) >= NY / 2) return -1;
+        return kx * nky + (ky >= 0 ? ky : ky + nky);
+    };
+    std::vector<char> done(size_t(nkx) * nky, 0);
+    for (int pass = 0; pass < 2; ++pass)   // first the wavenumbers whose partners are all kept
+        for (int kx = 0; kx < nkx; ++kx)
+            for (int ky = -(NY / 2 - 1); ky < NY / 2; ++ky) {
+                const int s = index(kx, ky);
+                if (done[s] || (pass == 0 && (kx == 0 || ky < 0))) continue;
+                done[s] = 1;
+                f.rep.push_back(s);
+                f.mem.push_back(s);
+                for (auto [px, py] : partners(kx, ky)) {
+                    const int o = kx == 0 && ky == 0 ? -1 : index(px, py);
+                    const bool take = o >= 0 && !done[o];
+                    if (take) done[o] = 1;
+                    f.mem.push_back(take ? o : -1);
+                }
+            }
+    return f;
 }
 
 // Structural blocks (see SystemTables::nblk): union-find over rows (0..n-1)

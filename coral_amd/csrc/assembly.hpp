@@ -84,8 +84,8 @@ struct SystemTables {
     std::vector<int> blk_row, blk_col;   // [nblk][nblk_n]
     int band_width() const { return nl + nu + 1; }
     // Symmetries of the operators between wavenumbers: where they exist, the
-    // system at k' = (kx, -ky) (SYM_REFLECT) or k' = (ky, -kx) (SYM_ROTATE, for
-    // equal box lengths) is that at k with rows and columns renumbered and some
+    // system at k' = (kx, -ky) (reflect) or k' = (ky, -kx) (rotate, for equal box
+    // lengths) is that at k with rows and columns renumbered and some
     // signs changed: A(k')(row[i], col[j]) = rsign[i] csign[j] A(k)(i, j) for M and
     // L alike, so one factorization serves both wavenumbers.
     struct Symmetry {
@@ -95,6 +95,20 @@ struct SystemTables {
     };
     Symmetry reflect, rotate;
 };
+
+// Which wavenumbers of a kxky system share one factorization (index ix * (NY - 1)
+// + jy, ky = jy below NY / 2 and jy - (NY - 1) from there on): rep[r] is factored
+// and serves mem[r * nslot + q], q < nslot, the first of them itself, the q-th at
+// its symmetry sym[q - 1] (-1: none).  With the reflection, (kx, ky) and (kx, -ky)
+// share; with the rotation (boxes of equal lengths only), (kx, ky) and (ky, -kx);
+// with both, those four and (ky, kx).  The (0, 0) system is the identity and
+// stands alone.  nslot = 1 and empty arrays: nothing is shared.
+struct FactorSharing {
+    int nslot = 1;
+    std::vector<int> rep, mem;
+    std::vector<SystemTables::Symmetry> sym;
+};
+FactorSharing factor_sharing(const SystemTables &t, int nkx, int NY, bool square_box);
 
 // Extraction of a full-variable term: Chebyshev coefficient n of the term is
 // sum_{k in [rowptr[n], rowptr[n+1])} val[k] * state[col[k]], times the

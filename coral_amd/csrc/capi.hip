@@ -6,7 +6,6 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -342,72 +341,23 @@ FFTPlan make_plan(int N, DevBuf<double2> &tw) {
     return p;
 }
 
-// Which wavenumbers share factors (SystemTables::Symmetry): d.rep_h the systems
-// factored, d.mem the systems each serves, syms the symmetry of slots 1 .. .
-// With the reflection, (kx, ky) and (kx, -ky) share; with the rotation, (kx, ky)
-// and (ky, -kx), which needs equal box lengths; with both, those four and
-// (ky, kx).  Factors are two thirds of what a solve reads.  The (0, 0) system is
-// the identity and stands alone.  CORAL_AMD_NO_SHARED_FACTORS=1 before
-// coral_amd_create factors every system.
+// Which wavenumbers share factors: d.rep_h the systems factored, d.mem the systems
+// each serves, syms the symmetry of slots 1 .. .  Factors are two thirds of what a
+// solve reads.  CORAL_AMD_NO_SHARED_FACTORS=1 before coral_amd_create factors
+// every system.
 void share_factors(SysDev &d, const KeptModes &km, std::vector<Solve16Sym> &syms) {
-    const SystemTables &t = *d.t;
     const char *off = std::getenv("CORAL_AMD_NO_SHARED_FACTORS");
     if (off && off[0] == '1') return;
-    const bool refl = t.reflect.found, rota = t.rotate.found && km.kx_box == km.ky_box;
-    if (!refl && !rota) return;
-    auto as_sym = [](const SystemTables::Symmetry &y) { return Solve16Sym{y.row, y.col, y.rneg, y.cneg}; };
-    const int nslot = refl && rota ? 4 : 2;
     // (two right-hand sides' word tables fit the solve's LDS)
     if (2 * size_t(d.nblk) * (d.blk_n + 2 * SOLVE16_WPAD) * sizeof(unsigned) > 32768) return;
-    typedef std::pair<int, int> K;
-    const std::function<K(K)> F = [](K k) { return K(k.first, -k.second); }, R = [](K k) { return K(k.second, -k.first); };
-    std::vector<std::function<K(K)>> ops;
-    if (refl) {
-        ops.push_back(F);
-        syms.push_back(as_sym(t.reflect));
-    }
-    if (rota) {
-        ops.push_back(R);
-        syms.push_back(as_sym(t.rotate));
-    }
-    if (nslot == 4) {
-        // the reflection after the rotation: (ky, kx)
-        ops.push_back([&](K k) { return F(R(k)); });
-        Solve16Sym c = as_sym(t.rotate);
-        for (int i = 0; i < t.total; ++i) {
-            c.rneg[i] ^= t.reflect.rneg[c.row[i]];
-            c.cneg[i] ^= t.reflect.cneg[c.col[i]];
-            c.row[i] = t.reflect.row[c.row[i]];
-            c.col[i] = t.reflect.col[c.col[i]];
-        }
-        syms.push_back(c);
-    }
-    auto index = [&](K k) -> int {
-        if (k.first < 0 || k.first >= km.nkx || std::abs(k.second) >= km.NY / 2) return -1;
-        return k.first * km.nky + (k.second >= 0 ? k.second : k.second + km.NY - 1);
-    };
-    std::vector<char> done(d.nsys, 0);
-    std::vector<int> mem;
-    for (int pass = 0; pass < 2; ++pass)   // first the wavenumbers whose partners are all kept
-        for (int kx = 0; kx < km.nkx; ++kx)
-            for (int ky = -(km.NY / 2 - 1); ky < km.NY / 2; ++ky) {
-                const K k(kx, ky);
-                const int s = index(k);
-                if (done[s] || (pass == 0 && (kx == 0 || ky < 0))) continue;
-                done[s] = 1;
-                d.rep_h.push_back(s);
-                mem.push_back(s);
-                for (int q = 1; q < nslot; ++q) {
-                    const int o = kx == 0 && ky == 0 ? -1 : index(ops[q - 1](k));
-                    const bool take = o >= 0 && !done[o];
-                    if (take) done[o] = 1;
-                    mem.push_back(take ? o : -1);
-                }
-            }
-    d.nslot = nslot;
-    d.nrep = int(d.rep_h.size());
-    d.rep.upload(d.rep_h);
-    d.mem.upload(mem);
+    const FactorSharing f = factor_sharing(*d.t, km.nkx, km.NY, km.kx_box == km.ky_box);
+    if (f.nslot == 1) return;
+    for (auto &y : f.sym) syms.push_back(Solve16Sym{y.row, y.col, y.rneg, y.cneg});
+    d.nslot = f.nslot;
+    d.rep_h = f.rep;
+    d.nrep = int(f.rep.size());
+    d.rep.upload(f.rep);
+    d.mem.upload(f.mem);
 }
 
 void fill_system_device(SysDev &d, int nstages, const KeptModes &km, hipStream_t st, int NZ) {

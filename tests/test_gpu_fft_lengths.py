@@ -10,8 +10,7 @@ from conftest import product_recipe
 
 pytestmark = pytest.mark.gpu
 
-# 3 N / 2 = 24, 27, 36, ... points; the deep grids have enough lines for the
-# wide plans of the short lengths, the shallow ones take the thin plans
+# 3 N / 2 = 24, 27, 36, ... points, on shallow grids and (the short lengths) deep ones
 GRIDS = [(16, 18, 17), (18, 16, 17), (24, 16, 20), (32, 24, 17), (36, 32, 17), (48, 36, 17), (54, 48, 17),
          (64, 54, 17), (72, 64, 17), (96, 72, 17), (108, 96, 17), (128, 108, 17), (144, 128, 17), (162, 144, 17),
          (192, 162, 17), (216, 192, 17), (16, 216, 65), (16, 72, 129), (18, 72, 129), (24, 96, 129), (32, 96, 97),
@@ -62,3 +61,35 @@ def test_products_and_transforms_match_oracle(native_lib, grid):
     for a, b in zip(fields, ora.physical_full_variables()):
         assert rel(a, b) <= tol
     assert abs(cfl - ora.cfl_dt) <= 1e-9 * abs(ora.cfl_dt)
+
+
+# lengths that share a transform between two lines scaled apart: several lines
+# per wavefront (27, 108, 216), one (288, 486), two wavefronts per line (648)
+@pytest.mark.parametrize("small", ["t", "w"])
+@pytest.mark.parametrize("grid", [(18, 16, 17), (72, 48, 17), (144, 16, 17), (192, 16, 17), (324, 16, 17), (432, 16, 17)],
+                         ids=lambda g: "x".join(map(str, g)))
+def test_small_lines_keep_their_digits(native_lib, grid, small):
+    """A variable of 1e-8 of the others (and its products beside theirs) comes out
+    as accurate as the others: the lines of a pair are scaled by powers of two of
+    their own.  Without that its errors would be 1e-8 of its size."""
+    from coral_amd import solver
+    NX, NY, NZ = grid
+    print("grid", grid, small, flush=True)
+    r = product_recipe("coral.equations.rbc_ra1e5")
+    geo = O.Geometry(NX, NY, NZ, 2 * np.pi, 2 * np.pi)
+    ora = O.OracleSolver(r, geo, "ARS_222")
+    rng = np.random.default_rng(NX)
+    k = rng.standard_normal(ora.field[0].shape) + 1j * rng.standard_normal(ora.field[0].shape)
+    ops, v = ora.kops[0], r.kxky_systems[0].var_names.index(small)
+    k[..., ops.posP[ops.var_first[v]:ops.var_first[v] + ops.var_size[v]]] *= 1e-8
+    k[~ora.keep] = 0.0
+    k[0, 0] = 0.0
+    O.project_kx0_plane(k, geo)
+    ora.field, ora.zfield = [k.copy()], [0.0 * z for z in ora.zfield]
+    q = ora.quad_spectra(ora.field, ora.zfield)
+    with solver.Solver(r, NX, NY, NZ, 2 * np.pi, 2 * np.pi) as g:
+        g.set_state([k], ora.zfield)
+        got = g.products()
+    for i, s in enumerate(q):
+        want = np.where(ora.keep[:, :, None], s, 0.0)
+        assert np.linalg.norm(got[i] - want) <= 2e-14 * np.linalg.norm(want), i   # the bar of the test above

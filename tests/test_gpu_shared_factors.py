@@ -76,3 +76,49 @@ def test_shared_factors_match_factoring_every_system(native_lib, monkeypatch, ca
     per = np.linalg.norm(x - x1, axis=-1) / np.maximum(np.linalg.norm(x1, axis=-1), 1e-300)
     assert per.max() <= 1e-8, np.unravel_index(per.argmax(), per.shape)
     assert np.linalg.norm(s - s1) <= 1e-10 * np.linalg.norm(s1)
+
+
+# recipe, NX = NY, NZ, whole systems (16 subdiagonals), complex factors: every
+# window size (2, 3, 4 registers) and both element types with two right-hand
+# sides per wavefront, which takes 1024 of such wavefronts
+TWO = [
+    ("radiative_heating.coral.equations", 96, 14, False, False),
+    ("radiative_heating.coral.equations", 96, 14, False, True),
+    ("coral.equations.rbc_ra1e5", 96, 14, False, True),
+    ("coral.equations.rbc_ra1e5", 144, 14, True, False),
+    ("coral.equations.rbc_ra1e5", 144, 14, True, True),
+    ("coral.equations.rrbc_ra5e7_ek1e-4", 144, 14, True, True),
+]
+
+
+@pytest.mark.parametrize("case", TWO, ids=[f"{c[0].split('.')[-1]}-{c[1]}x{c[2]}{'w' * c[3]}{'c' * c[4]}" for c in TWO])
+def test_two_right_hand_sides_per_wavefront(native_lib, monkeypatch, case):
+    from coral_amd import solver
+    name, NX, NZ, whole, cplx = case
+    print("case", case, flush=True)
+    monkeypatch.setenv("CORAL_AMD_NO_BLOCK_SPLIT", "1" if whole else "0")
+    monkeypatch.setenv("CORAL_AMD_COMPLEX_FACTORS", "1" if cplx else "0")
+    from conftest import recipe
+    r = product_recipe(name) if name.startswith("coral.") else recipe(name)
+    rng = np.random.default_rng(11)
+    out, rhs = [], None
+    for off in ("0", "1"):
+        monkeypatch.setenv("CORAL_AMD_NO_SHARED_FACTORS", off)
+        with solver.Solver(r, NX, NX, NZ, 2.0, 2.0) as g:
+            g.factorize_operators(1e-5)
+            nfac, share = g.factored_systems(0)
+            nblk, _, kl, _ = g.factor_blocks(0)[:4]
+            if off == "0":
+                assert share >= 2 and (nfac * nblk + 3) // 4 * (share // 2) >= 1024
+                assert (kl == 16) == whole and g.factor_is_real(0) == (not cplx)
+                shape = (NX // 2, 3 * NX // 2, g.totals[0])
+                rhs = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+            else:
+                assert share == 1
+            out.append(g.solve_system(0, rhs))
+    x, x1 = out
+    # the bars of the test above
+    assert np.array_equal(x[0, 0], x1[0, 0])
+    assert np.linalg.norm(x - x1) <= 1e-10 * np.linalg.norm(x1)
+    per = np.linalg.norm(x - x1, axis=-1) / np.maximum(np.linalg.norm(x1, axis=-1), 1e-300)
+    assert per.max() <= 1e-8, np.unravel_index(per.argmax(), per.shape)
