@@ -30,8 +30,8 @@ HIP_FLAGS = [
 ]
 HOST_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall"]
 
-HIP_SOURCES = ["kernels.hip", "xpass.hip", "xpass_b.hip", "xpass_c.hip", "xpass_d.hip", "xpass_e.hip", "ypass.hip", "ztransform.hip", "capi.hip", "ztransform32.hip",
-               "noalloc.hip", "nn.hip"]
+HIP_SOURCES = ["kernels.hip", "xpass.hip", "xpass_b.hip", "xpass_c.hip", "xpass_d.hip", "xpass_e.hip", "ypass.hip",
+               "ztransform.hip", "capi.hip", "ztransform32.hip", "noalloc.hip", "nn.hip"]
 HOST_SOURCES = ["assembly.cpp"]
 
 

@@ -469,10 +469,9 @@ void fill_system_device(SysDev &d, int nstages, const KeptModes &km, hipStream_t
     const int kv = t.nl + t.nu;
     const char *force = std::getenv("CORAL_AMD_COMPLEX_FACTORS");
     d.real = t.real_form && !(force && force[0] == '1');
-    // 16-lane solve layout when the band allows it; U arrays padded (zeroed) on
-    // both sides for its out-of-record reads
-    // (records of four matrices interleaved, in groups of four and blocks of 16
-    // columns; the slots past the last matrix stay zero).  The 16-lane layout
+    // 16-lane solve layout when the band allows it (records of four matrices
+    // interleaved, in groups of four and blocks of 16 columns; the slots past the
+    // last matrix stay zero).  The 16-lane layout
     // factors the structural blocks of the operator separately when it splits
     // (CORAL_AMD_NO_BLOCK_SPLIT=1 keeps whole systems).
     const char *nosplit = std::getenv("CORAL_AMD_NO_BLOCK_SPLIT");
@@ -511,7 +510,7 @@ void fill_system_device(SysDev &d, int nstages, const KeptModes &km, hipStream_t
     const size_t lsize = d.ncol16 > 0 ? nmat4 * d.ncol16 * solve16_klp(d.blk_nl)
                                       : size_t(d.nsys) * t.total * std::max(t.nl, 1);
     const size_t usize =
-        (d.ncol16 > 0 ? nmat4 * nb * (bkv + 1) : size_t(d.nsys) * t.total * (kv + 1)) + 2 * size_t(SOLVE16_PAD);
+        d.ncol16 > 0 ? nmat4 * nb * (bkv + 1) : size_t(d.nsys) * t.total * (kv + 1);
     if (d.real) {
         d.Lr.alloc(lsize);
         d.Ur.alloc(usize);
@@ -557,10 +556,10 @@ void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
         a.km = d.kxky ? c.km : KeptModes{1, 1, 2, 0.0, 0.0};
         a.work = work.p;
         a.Lf = d.Lf.p;
-        a.Uf = d.Uf.p ? d.Uf.p + SOLVE16_PAD : nullptr;
+        a.Uf = d.Uf.p;
         a.rot = d.real ? d.rot.p : nullptr;
         a.Lr = d.Lr.p;
-        a.Ur = d.Ur.p ? d.Ur.p + SOLVE16_PAD : nullptr;
+        a.Ur = d.Ur.p;
         a.ncol16 = d.ncol16;
         a.nblk = d.nblk;
         a.blk_n = d.blk_n;
@@ -575,7 +574,7 @@ void factorize(coral_amd_ctx &c, SysDev &d, double dt) {
     }
     if (d.ncol16 > 0) {
         const int bkv = d.blk_nl + d.blk_nu, elem = d.real ? 8 : 16, nb = 16 * ((d.blk_n + 15) / 16);
-        const void *Ufull = d.real ? (const void *)(d.Ur.p + SOLVE16_PAD) : (const void *)(d.Uf.p + SOLVE16_PAD);
+        const void *Ufull = d.real ? (const void *)d.Ur.p : (const void *)d.Uf.p;
         if (d.ulen.n < size_t(nb)) d.ulen.alloc(nb);
         std::vector<int2> ucol;
         solve16_ucol(c.stream, Ufull, elem, d.blk_n, bkv, nmat, d.ulen.p, ucol, &d.ustride);
@@ -1515,10 +1514,10 @@ void solve_system(coral_amd_ctx &c, SysDev &d, const double2 *rhs, double2 *out,
         if (solve16_args_of(c, d, rhs, out, sa)) {
             done = d.real ? launch_solve16_real(c.stream, sa) : launch_solve16_complex(c.stream, sa);
         } else if (d.real)
-            launch_solve_real(c.stream, d.Lr.p, d.Ur.p + SOLVE16_PAD, d.piv.p, d.rot.p, id0, t.total, t.nl, kv,
+            launch_solve_real(c.stream, d.Lr.p, d.Ur.p, d.piv.p, d.rot.p, id0, t.total, t.nl, kv,
                               d.nsys, rhs, out);
         else
-            launch_solve(c.stream, d.Lf.p, d.Uf.p + SOLVE16_PAD, d.piv.p, t.total, t.nl, kv, d.nsys, rhs, out);
+            launch_solve(c.stream, d.Lf.p, d.Uf.p, d.piv.p, t.total, t.nl, kv, d.nsys, rhs, out);
         if (!done) throw std::runtime_error("16-lane solve rejected a band it was factored for");
     });
 }
@@ -2555,20 +2554,20 @@ int coral_amd_banded_solve(int32_t device, int32_t n, int32_t kl, int32_t ku, in
             DevBuf<int2> ucol;
             DevBuf<unsigned> words;
             L16.alloc(nmat4 * ncol16 * solve16_klp(kl));
-            Uf.alloc(nmat4 * nb * (kv + 1) + 2 * size_t(SOLVE16_PAD));
+            Uf.alloc(nmat4 * nb * (kv + 1));
             piv.alloc(size_t(nsys) * nb);
             HIP_OK(hipMemsetAsync(L16.p, 0, L16.n * sizeof(double2), st));
             HIP_OK(hipMemsetAsync(Uf.p, 0, Uf.n * sizeof(double2), st));
             HIP_OK(hipMemsetAsync(piv.p, 0, piv.n, st));
-            launch_factor_lapack16(st, work.p, n, kl, ku, nsys, ncol16, L16.p, Uf.p + SOLVE16_PAD, piv.p, inf.p);
+            launch_factor_lapack16(st, work.p, n, kl, ku, nsys, ncol16, L16.p, Uf.p, piv.p, inf.p);
             ulen.alloc(nb);
             std::vector<int2> uc;
             long long ustride = 0;
-            solve16_ucol(st, Uf.p + SOLVE16_PAD, 16, n, kv, nsys, ulen.p, uc, &ustride);
+            solve16_ucol(st, Uf.p, 16, n, kv, nsys, ulen.p, uc, &ustride);
             Ut.alloc(size_t((nsys + 3) / 4) * size_t(ustride));
             HIP_OK(hipMemsetAsync(Ut.p, 0, Ut.n * sizeof(double2), st));
             ucol.upload(uc);
-            solve16_trim_u_copy(st, Uf.p + SOLVE16_PAD, 16, n, kv, nsys, ucol.p, ustride, Ut.p);
+            solve16_trim_u_copy(st, Uf.p, 16, n, kv, nsys, ucol.p, ustride, Ut.p);
             words.upload(solve16_words(n, 1, n, nullptr, nullptr, nullptr));
             rb.alloc(size_t(nsys) * n);
             sink.alloc(64);

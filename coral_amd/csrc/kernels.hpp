@@ -288,9 +288,10 @@ void launch_factor(hipStream_t st, const FactorArgs &a);
 void launch_factor_lapack(hipStream_t st, double2 *work, int n, int kl, int ku, int nsys, double2 *Lf, double2 *Uf,
                           unsigned char *piv, int *info);
 // the same factorization into the records of the 16-lane solve (ncol16 =
-// solve16_ncol(n, kl, kl + ku) > 0): L16 [ceil(nsys/4)*4][ncol16][kl],
-// Ufull with SOLVE16_PAD elements before it, pivots [nsys][16*ceil(n/16)];
-// all three cleared by the caller
+// solve16_ncol(n, kl, kl + ku) > 0, the layout at split_factors16): L16
+// [ceil(nsys/4)][ncol16][4][solve16_klp(kl)], Ufull
+// [ceil(nsys/4)][16*ceil(n/16)][4][kl + ku + 1], pivots [nsys][16*ceil(n/16)]; all
+// three cleared by the caller
 void launch_factor_lapack16(hipStream_t st, double2 *work, int n, int kl, int ku, int nsys, int ncol16, double2 *L16,
                             double2 *Ufull, unsigned char *piv, int *info);
 void launch_solve(hipStream_t st, const double2 *Lf, const double2 *Uf, const unsigned char *piv, int n, int kl,
@@ -303,10 +304,6 @@ int solve16_ncol(int n, int kl, int kv);
 // in kernels.hip), and the entries per multiplier record, one per window slot
 __host__ __device__ inline int solve16_window(int kl) { return kl < 16 ? kl + 1 : 16; }
 __host__ __device__ inline int solve16_klp(int kl) { return solve16_window(kl); }
-// U arrays of the solves carry this many elements of padding on each side (the
-// 16-lane solve reads up to 16 elements before the first record and 64 past
-// the last)
-constexpr int SOLVE16_PAD = 2048;
 // columns before the first in the solve's table of trimmed U records: the
 // backward sweep fetches that many steps ahead
 constexpr int SOLVE16_UPAD = 8;

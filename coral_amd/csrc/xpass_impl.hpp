@@ -1,5 +1,5 @@
 // x pass of the nonlinear step on wavefront FFTs: templates and radix plans
-// (xpass.hip and xpass_b.hip .. xpass_d.hip instantiate them over the lengths).
+// (xpass.hip and xpass_b.hip .. xpass_e.hip instantiate them over the lengths).
 //
 // For each line: inverse real FFTs of the full variables (two real lines are
 // packed into one complex sequence, f0 + i f1), the quadratic products and
