@@ -239,10 +239,12 @@ __device__ inline T bal_scale(unsigned mbits) { return bal_pow<T>(mbits, -1); }
 // that is not taken otherwise; the empty asm keeps it from being turned into a
 // select per value), and the scaling back makes every value of the line a NaN.
 // Costs 1 % of the pass: us per launch 753 -> 759 at 288^2 x 97, 233 -> 236 at
-// 192^2 x 65, 26.5 -> 27.0 at 72 x 48 x 41.
+// 192^2 x 65, 26.5 -> 27.0 at 72 x 48 x 41.  FP64 only: the lines of the FP32
+// chain share their transforms at every length, as those of the five FP64
+// lengths that do not balance do.
 template <class T>
 __device__ inline bool bal_bad(unsigned mbits) {
-    return mbits >= (sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u);
+    return sizeof(T) == 8 && mbits >= 0x7ff00000u;
 }
 template <class T>
 __device__ inline T bal_unscale(unsigned mbits) {
