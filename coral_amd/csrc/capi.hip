@@ -144,14 +144,17 @@ struct coral_amd_ctx {
     Problem P;
     int device = 0;
     hipStream_t stream = nullptr;
-    // the mean systems' NL terms, right-hand sides and solves run on side
-    // streams (mean system k on stream k mod NSIDE, so that their chains of
-    // small kernels run beside each other too), overlapped with the kxky work:
-    // they wait for Qhat (ev_qhat) and the kxky side waits for their solutions
-    // (ev_mean) before the next stage's mean extraction
-    static constexpr int NSIDE = 2;
-    hipStream_t side[NSIDE] = {};
-    hipEvent_t ev_qhat = nullptr, ev_mean[NSIDE] = {};
+    // the mean systems' NL terms, right-hand sides and solves run on a second
+    // stream (none without mean systems), overlapped with the kxky work: they
+    // wait for Qhat (ev_qhat) and the kxky side waits for their solutions
+    // (ev_mean) before the next stage's mean extraction.  A third stream, so that
+    // two mean systems' chains of small kernels run beside each other too, was no
+    // gain: us per step as graph replays 289 with it and 282 without at
+    // 64 x 64 x 33, 189 and 187 at 24 x 16 x 17, 563 and 555 at 96 x 96 x 48 (eager
+    // 275 and 280, 201 and 203, 548 and 536), 48 runs as one ensemble 38.3 and
+    // 39.6 steps/s, and a run took 0.2 ms more to make and end.
+    hipStream_t side = nullptr;
+    hipEvent_t ev_qhat = nullptr, ev_mean = nullptr;
     bool mean_pending = false;
     KeptModes km{};
     std::vector<std::unique_ptr<SysDev>> ks, zs;
@@ -268,10 +271,8 @@ struct coral_amd_ctx {
         }
         drop_graphs();
         if (ev_qhat) (void)hipEventDestroy(ev_qhat);
-        for (auto &e : ev_mean)
-            if (e) (void)hipEventDestroy(e);
-        for (auto &st : side)
-            if (st) (void)hipStreamDestroy(st);
+        if (ev_mean) (void)hipEventDestroy(ev_mean);
+        if (side) (void)hipStreamDestroy(side);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -695,11 +696,10 @@ void nl_assemble(coral_amd_ctx &c, SysDev &d, double2 *Khat) {
     c.timed(d.kxky ? "nl_assemble" : "nl_mean", [&] { launch_nl(c.stream, a); });
 }
 
-// the main stream waits for the mean systems' pending work on the side streams
+// the main stream waits for the mean systems' pending work on the side stream
 void join_mean(coral_amd_ctx &c) {
     if (!c.mean_pending) return;
-    for (size_t k = 0; k < std::min<size_t>(c.zs.size(), c.NSIDE); ++k)
-        HIP_OK(hipStreamWaitEvent(c.stream, c.ev_mean[k], 0));
+    HIP_OK(hipStreamWaitEvent(c.stream, c.ev_mean, 0));
     c.mean_pending = false;
 }
 
@@ -715,17 +715,17 @@ void swap_step_buffers(coral_amd_ctx &c) {
     ++c.nswap;
 }
 
-// f's launches (and timer events) go to side stream k
+// f's launches (and timer events) go to the side stream
 template <class F>
-void on_side(coral_amd_ctx &c, int k, F &&f) {
-    std::swap(c.stream, c.side[k]);
+void on_side(coral_amd_ctx &c, F &&f) {
+    std::swap(c.stream, c.side);
     try {
         f();
     } catch (...) {
-        std::swap(c.stream, c.side[k]);
+        std::swap(c.stream, c.side);
         throw;
     }
-    std::swap(c.stream, c.side[k]);
+    std::swap(c.stream, c.side);
 }
 
 // Chebyshev coefficients of all full variables from the given states, then the
@@ -1576,7 +1576,7 @@ void project_kx0(coral_amd_ctx &c) {
 // x^{n+1} = x_s.
 // A step in phases (one_step_beyond, PL_IMEX_timestepping_marching.f90:3-48):
 // step_begin (the stage coefficients), per stage stage_nl (NL terms, the mean
-// systems on the side streams) and per kxky system stage_rhs then
+// systems on the side stream) and per kxky system stage_rhs then
 // stage_solve, and step_end.  one_step runs them for one run; the ensemble's
 // lockstep step runs every run's stage_nl and stage_rhs, then their solves
 // as one launch.
@@ -1637,24 +1637,24 @@ void stage_solve(coral_amd_ctx &c, int i, SysDev &d) {
     if (c.refine == 2 || (c.refine == 1 && i == s - 1)) refine_solution(c, d, d.R.p, d.X[i]->p, c.P.a_arr[i * s + i]);
 }
 
-// stage i's NL terms, and the mean systems' whole stage on the side streams
+// stage i's NL terms, and the mean systems' whole stage on the side stream
 void stage_nl(coral_amd_ctx &c, int i) {
     std::vector<const double2 *> kst, zst;
     for (auto &d : c.ks) kst.push_back(i == 0 ? d->field.p : d->X[i - 1]->p);
     for (auto &d : c.zs) zst.push_back(i == 0 ? d->field.p : d->X[i - 1]->p);
     nl_terms(c, kst, zst, i);
-    const int nz = int(c.zs.size());
-    for (int k = 0; k < nz; ++k)
-        on_side(c, k % c.NSIDE, [&] {
-            SysDev &d = *c.zs[k];
+    if (c.zs.empty()) return;
+    on_side(c, [&] {
+        HIP_OK(hipStreamWaitEvent(c.stream, c.ev_qhat, 0));
+        for (auto &d : c.zs) {
             // NL terms from the Qhat of nl_terms
-            if (k < c.NSIDE) HIP_OK(hipStreamWaitEvent(c.stream, c.ev_qhat, 0));
-            nl_assemble(c, d, d.Khat[i]->p);
-            stage_rhs(c, i, d);
-            stage_solve(c, i, d);
-            if (k + c.NSIDE >= nz) HIP_OK(hipEventRecord(c.ev_mean[k % c.NSIDE], c.stream));
-        });
-    c.mean_pending = nz > 0;
+            nl_assemble(c, *d, d->Khat[i]->p);
+            stage_rhs(c, i, *d);
+            stage_solve(c, i, *d);
+        }
+        HIP_OK(hipEventRecord(c.ev_mean, c.stream));
+    });
+    c.mean_pending = true;
 }
 
 void step_end(coral_amd_ctx &c) {
@@ -1675,8 +1675,8 @@ void one_step(coral_amd_ctx &c) {
     step_end(c);
 }
 
-// Two graphs of one step each, captured from the stream (the side streams
-// join through their events).  Capturing runs one_step's host logic, which
+// Two graphs of one step each, captured from the stream (the side stream
+// joins through its events).  Capturing runs one_step's host logic, which
 // swaps the step buffers; after both captures they are back where they were.
 // The step holds no memset and no allocation, so the graphs replay it
 // exactly; they are dropped when dt changes.
@@ -1869,12 +1869,9 @@ int coral_amd_create(const coral_amd_problem *prob, int device, coral_amd_ctx **
         c->device = device;
         HIP_OK(hipSetDevice(device));
         HIP_OK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-        // (as many side streams as mean systems use: one costs 0.1 to 3 ms to
-        // make and 0.3 to destroy)
-        for (size_t k = 0; k < std::min<size_t>(P.zero.size(), c->NSIDE); ++k)
-            HIP_OK(hipStreamCreateWithFlags(&c->side[k], hipStreamNonBlocking));
+        if (!P.zero.empty()) HIP_OK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
         HIP_OK(hipEventCreateWithFlags(&c->ev_qhat, hipEventDisableTiming));
-        for (auto &e : c->ev_mean) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIP_OK(hipEventCreateWithFlags(&c->ev_mean, hipEventDisableTiming));
         c->km = KeptModes{P.nkx, P.nky, P.NY, P.kx_box, P.ky_box};
         for (auto &t : P.kxky) {
             c->ks.emplace_back(new SysDev());
@@ -1998,8 +1995,7 @@ int coral_amd_upload_state(coral_amd_ctx *c, int32_t kind, int32_t isys, const d
         // the copies below go through the null stream, which does not wait
         // for the context's non-blocking streams: finish queued steps first
         HIP_OK(hipStreamSynchronize(c->stream));
-        for (auto &st : c->side)
-            if (st) HIP_OK(hipStreamSynchronize(st));
+        if (c->side) HIP_OK(hipStreamSynchronize(c->side));
         if (kind == 0) {
             if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
             SysDev &d = *c->ks[isys];
@@ -2620,8 +2616,7 @@ int coral_amd_system_solve(coral_amd_ctx *c, int32_t isys, const double *rhs, do
         if (isys < 0 || isys >= int(c->ks.size())) throw std::runtime_error("bad kxky system index");
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        for (auto &st : c->side)
-            if (st) HIP_OK(hipStreamSynchronize(st));
+        if (c->side) HIP_OK(hipStreamSynchronize(c->side));
         SysDev &d = *c->ks[isys];
         const int total = d.t->total;
         upload_modes(*c, rhs, total, d.R.p);
@@ -2677,8 +2672,7 @@ int coral_amd_set_precision(coral_amd_ctx *c, int32_t mode, int32_t refine) {
             throw std::runtime_error("fixed physical fields and the Smagorinsky viscosity run with the FP64 transform chain only");
         HIP_OK(hipSetDevice(c->device));
         HIP_OK(hipStreamSynchronize(c->stream));
-        for (auto &st : c->side)
-            if (st) HIP_OK(hipStreamSynchronize(st));
+        if (c->side) HIP_OK(hipStreamSynchronize(c->side));
         Problem &P = c->P;
         if (mode == 1 && !c->spec32.p) {
             ZFrags32 zf;
@@ -3356,7 +3350,7 @@ bool ens_lockstep_ok(const coral_amd_ensemble &e, std::string *why = nullptr) {
 }
 
 // The lockstep graphs (one per buffer assignment): per stage every run's NL
-// terms (its mean systems forked onto its side streams) and kxky right-hand
+// terms (its mean systems forked onto its side stream) and kxky right-hand
 // sides, then the stage's kxky solves grouped by kernel variant, each group
 // one k_solve16_batch launch; systems the 16-lane solve does not take are
 // solved on their own.  Every run's arithmetic is its own step's.
