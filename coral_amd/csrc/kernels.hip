@@ -1744,15 +1744,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // block of 16 at a time, and entries outside a record read as zero through its
 // buffer descriptor.  (With the table in LDS and the bounds in vector
 // registers a step waited for an LDS read and a quarter-rate multiply, and the
-// kernel held 137 VGPRs, now 86.)
+// kernel held 137 VGPRs, now 88 with one right-hand side and 119 with two.)
 // Small grids are bound by the chain of steps of one wavefront: 64 x 64 x 33
-// 43 -> 31 us per launch, 72 x 48 x 41 54 -> 37, over both sweeps.  From
+// 43 -> 35 us per launch, 72 x 48 x 41 53 -> 40, over both sweeps.  From
 // 128^2 x 65 on a launch with factors of its own for every system moves its
-// bytes at 4.0 to 4.4 TB/s, what a device copy reaches (256^2 x 129: 1.51 ms);
-// sharing factors between related systems takes 1.51 -> 0.87 ms there with two
-// systems each (the rotating recipe), 0.85 with four (the non-rotating one),
-// 0.44 -> 0.25 at 192^2 x 65, 0.21 -> 0.14 at 128^2 x 65, bound by the vector
-// instructions of the steps.
+// bytes at 4.0 to 4.4 TB/s, close to a device copy (256^2 x 129: 1.57 ms).
+// Sharing factors between related systems takes 1.57 -> 0.97 ms there with two
+// systems each (the rotating recipe; 4.6 GB at copy speed), 0.86 with four (3.6
+// GB at 4.2 TB/s: the vector instructions issue for 0.40 ms, and four wavefronts
+// per SIMD leave memory latency), 0.46 -> 0.25 at 192^2 x 65, 0.22 -> 0.14 at
+// 128^2 x 65.
 // ---------------------------------------------------------------------------
 // row_newbcast writes every lane of the row, so no old value is needed
 template <int T_>
