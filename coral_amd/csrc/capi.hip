@@ -1750,7 +1750,8 @@ void transpose(hipStream_t st, const TI *in, int R, int C, size_t ir, size_t ib,
 struct HostLayout {
     double2 *p;
     DevBuf<double2> own;
-    HostLayout(coral_amd_ctx &c, size_t n) {
+    hipStream_t st;
+    HostLayout(coral_amd_ctx &c, size_t n) : st(c.stream) {
         if (c.H.n >= n) {
             p = c.H.p;
         } else if (c.G.n >= n) {
@@ -1759,6 +1760,10 @@ struct HostLayout {
             own.alloc(n);
             p = own.p;
         }
+    }
+    // what is queued on the stream may still read the array
+    ~HostLayout() {
+        if (own.p) (void)hipStreamSynchronize(st);
     }
 };
 

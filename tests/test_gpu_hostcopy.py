@@ -86,3 +86,30 @@ def test_reading_keeps_no_device_memory(native_lib):
         # the allocator hands out memory in pieces of up to 4 MiB; the spectra of
         # the nine products in the host's layout are 42 MB
         assert start - _free_bytes() <= volume + (8 << 20)
+
+
+def test_recipe_without_products(native_lib):
+    """One full variable and no products: the spectra are too small for a volume
+    in the host's layout, which then has an array of its own."""
+    from coral_amd import solver
+
+    from conftest import recipe
+    rng = np.random.default_rng(6)
+    out = []
+    for few in (False, True):
+        r = recipe("heat_equation.coral.equations")
+        if few:
+            r.full_vars, r.quad_vars = r.full_vars[:1], []
+            for s in r.kxky_systems + r.zero_systems:
+                s.nl = []
+        with solver.Solver(r, 32, 24, 33, 2.0, 3.0) as g:
+            if not out:
+                shape = (16, 36, g.totals[0])
+                a = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+                a[0] = 0.0
+            g.set_field("kxky", 0, a)
+            v = g.variable_physical("kxky", 0, 0)
+            g.set_variable_physical("kxky", 0, 0, 2.0 * v)
+            out.append((v, g.get_field("kxky", 0), g.bwd_transform(g.fwd_transform(v))))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y) and np.abs(x).max() > 0
